@@ -612,8 +612,8 @@ def main() -> int:
                     help="bounce rays in primary order or grouped by direction octant (vrt_bounce_generate_ex); "
                          "auto: timed after warm-up with the block orders")
     ap.add_argument("--anchor", default="sector", choices=["floor", "sector"],
-                    help="integer world origin of the camera rays: the camera's sector corner (default; the "
-                         "aligned-origin step) or floor(eye)")
+                    help="integer world origin of the camera rays: the camera's sector corner (default) or "
+                         "floor(eye)")
     ap.add_argument("--event-every", type=int, default=8,
                     help="HIP events around the launches of every n-th timed step (the roofline's launch times)")
     ap.add_argument("--only", default="all", choices=["all", "batched", "diff", "c1", "c3", "extras"],

@@ -270,9 +270,8 @@ class CameraSpec:
     anchor: the rays' integer world origin W (eye = pos - W, rounded to f32):
       "floor"   floor(pos), the reference's choice (eye in [0, 1));
       "sector"  floor(pos) rounded down to a multiple of 32 per axis, the corner of the camera's
-                sector (eye in [0, 32)): the casts take their aligned-origin step, 3 VALU
-                instructions shorter;
-      "zero"    0, world-space rays: the step also drops the additions of W (6 shorter).
+                sector (eye in [0, 32));
+      "zero"    0, world-space rays.
     The rays are the same world rays up to the f32 rounding of the eye."""
 
     ANCHORS = ("floor", "sector", "zero")

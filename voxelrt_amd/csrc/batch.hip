@@ -17,6 +17,7 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <bit>
 #include <chrono>
 #include <cstdio>
 #include <cstring>
@@ -35,8 +36,13 @@ namespace vrt {
 struct BatchSegDev {
     uint32_t kind, cam, ray_offset, hit_offset, count, block_begin;
     int32_t W[3];
-    uint32_t pad;
+    uint32_t own_tile;  // camera segments: the camera's own tile is the tuned one
     const uint32_t* count_ptr;
+    // camera segments: tiles of the tuned size per row, the camera's own tile size, its tiles per
+    // row, and 1 / width and 1 / height
+    udiv32 across, cam_tw, cam_th;
+    uint32_t cam_across;
+    float inv_w, inv_h;
 };
 
 struct BatchArgs {
@@ -48,7 +54,7 @@ struct BatchArgs {
     const float* dx; const float* dy; const float* dz;
     HitsOut h;
     uint32_t max_iters;
-    uint32_t tile_w, tile_h;
+    uint32_t tile_shift_w, tile_shift_h;  // log2 of the tuned tile (64 pixels)
 };
 
 __device__ __forceinline__ uint32_t find_segment(const BatchArgs& a, uint32_t block) {
@@ -61,10 +67,9 @@ __device__ __forceinline__ uint32_t find_segment(const BatchArgs& a, uint32_t bl
 }
 
 // Index of pixel (px, py) in the camera's own ray order (inverse of tile_pixel).
-__device__ __forceinline__ uint32_t camera_order_index(const vrt_camera& c, uint32_t px, uint32_t py) {
-    uint32_t tx = px / c.tile_w, ty = py / c.tile_h;
-    return (ty * (c.width / c.tile_w) + tx) * (c.tile_w * c.tile_h) + (py - ty * c.tile_h) * c.tile_w +
-           (px - tx * c.tile_w);
+__device__ __forceinline__ uint32_t camera_order_index(const BatchSegDev& sg, uint32_t px, uint32_t py) {
+    const uint32_t tx = udiv(sg.cam_tw, px), ty = udiv(sg.cam_th, py), tw = sg.cam_tw.d, th = sg.cam_th.d;
+    return (ty * sg.cam_across + tx) * (tw * th) + (py - ty * th) * tw + (px - tx * tw);
 }
 
 struct LaneRay {
@@ -81,28 +86,22 @@ __device__ __forceinline__ LaneRay lane_ray(const BatchArgs& a, const BatchSegDe
     if (!lr.valid) return lr;
     if (sg.kind == VRT_SEG_CAMERA) {
         const vrt_camera& c = a.cams[sg.cam];
-        uint32_t px, py;
-        tile_pixel(local, c.width, a.tile_w, a.tile_h, px, py);
+        // the tuned tiles are a wave's 64 pixels, with sides that are powers of two
+        const uint32_t tile = local >> 6, in = local & 63u;
+        const uint32_t ty = udiv(sg.across, tile), tx = tile - ty * sg.across.d;
+        const uint32_t px = (tx << a.tile_shift_w) + (in & ((1u << a.tile_shift_w) - 1u));
+        const uint32_t py = (ty << a.tile_shift_h) + (in >> a.tile_shift_w);
         float d[3];
-        camera_ray(c.forward, c.right, c.up, 1.0f / (float)c.width, 1.0f / (float)c.height, px, py, d);
+        camera_ray(c.forward, c.right, c.up, sg.inv_w, sg.inv_h, px, py, d);
         ray_setup(st, c.eye[0], c.eye[1], c.eye[2], d[0], d[1], d[2], c.world_origin[0], c.world_origin[1],
                   c.world_origin[2]);
-        lr.out = sg.hit_offset + camera_order_index(c, px, py);
+        lr.out = sg.hit_offset + (sg.own_tile ? local : camera_order_index(sg, px, py));
     } else {
         uint32_t i = sg.ray_offset + local;
         ray_setup(st, a.ox[i], a.oy[i], a.oz[i], a.dx[i], a.dy[i], a.dz[i], sg.W[0], sg.W[1], sg.W[2]);
         lr.out = sg.hit_offset + local;
     }
     return lr;
-}
-
-// The origin kind of the segment's rays (the camera's world origin for camera segments).
-__device__ __forceinline__ int segment_origin(const BatchArgs& a, const BatchSegDev& sg) {
-    if (sg.kind == VRT_SEG_CAMERA) {
-        const vrt_camera& c = a.cams[sg.cam];
-        return origin_kind(c.world_origin[0], c.world_origin[1], c.world_origin[2]);
-    }
-    return origin_kind(sg.W[0], sg.W[1], sg.W[2]);
 }
 
 template <int RPL, bool COUNT>
@@ -121,9 +120,12 @@ __device__ __forceinline__ void trace_block(const WorldView& w, const BatchArgs&
         uint32_t local = (block - sg.block_begin) * (64 * RPL) + (uint32_t)k * 64 + lane;
         lr[k] = lane_ray(a, sg, count, local, st[k]);
         done[k] = !lr[k].valid;
-        tame = tame && (done[k] || ray_is_tame(st[k]));
+        if constexpr (RPL > 1) {
+            ray_exact_inverse(st[k]);
+            tame = tame && (done[k] || ray_is_tame(st[k]));
+        }
     }
-    bool wave_tame = __all(tame);
+    const bool wave_tame = RPL > 1 && __all(tame);
     bool hit[RPL];
     int32_t v[RPL][3];
     uint32_t slot[RPL];
@@ -133,8 +135,7 @@ __device__ __forceinline__ void trace_block(const WorldView& w, const BatchArgs&
         slot[k] = 0;
     }
     if constexpr (RPL == 1) {
-        if (!done[0])
-            hit[0] = ray_trace_wave(w, st[0], a.max_iters, v[0], slot[0], wave_tame, segment_origin(a, sg));
+        if (!done[0]) hit[0] = ray_trace_wave(w, st[0], a.max_iters, v[0], slot[0]);
     } else {
         // the lane's rays step in lockstep, so one counter caps them all
         for (uint32_t it = 0; it < a.max_iters; it++) {
@@ -333,6 +334,13 @@ static int create_plan(const vrt_world* world, const vrt_batch* b, const vrt_bat
             if ((uint64_t)c.width * c.height > 0xFFFFFF00ull)
                 return fail(VRT_ERR_INVALID_ARGUMENT, "batch: camera with more than 2^32 - 256 pixels");
             d.count = c.width * c.height;
+            d.across = make_udiv32(c.width / tun->tile_w);
+            d.cam_tw = make_udiv32(c.tile_w);
+            d.cam_th = make_udiv32(c.tile_h);
+            d.cam_across = c.width / c.tile_w;
+            d.own_tile = c.tile_w == tun->tile_w && c.tile_h == tun->tile_h ? 1u : 0u;
+            d.inv_w = 1.0f / (float)c.width;
+            d.inv_h = 1.0f / (float)c.height;
             if (g.count_ptr) return fail(VRT_ERR_INVALID_ARGUMENT, "batch: camera segments have a fixed count");
         } else if (g.kind == VRT_SEG_RAYS) {
             if (d.count && (!b->rays.ox || !b->rays.oy || !b->rays.oz || !b->rays.dx || !b->rays.dy || !b->rays.dz))
@@ -405,8 +413,8 @@ static int create_plan(const vrt_world* world, const vrt_batch* b, const vrt_bat
         a.h.pos_z = b->hits.pos + 2 * hit_space;
     }
     a.max_iters = b->max_iters;
-    a.tile_w = tun->tile_w;
-    a.tile_h = tun->tile_h;
+    a.tile_shift_w = (uint32_t)std::countr_zero(tun->tile_w);
+    a.tile_shift_h = (uint32_t)std::countr_zero(tun->tile_h);
     *out = p;
     return VRT_OK;
 }

@@ -70,12 +70,9 @@ __device__ __forceinline__ void store_result(const HitsOut& h, uint32_t i, const
     if (h.material_data) h.material_data[i] = hit ? (uint32_t)h.palette[rec.w & 0xFF] : 0u;
 }
 
-// Traces one ray to completion.
-__device__ __forceinline__ void trace_full(const WorldView& w, RayState& st, uint32_t max_iters, bool wave_tame,
-                                           int origin, float& t, int4& rec) {
-    int32_t v[3];
-    uint32_t slot;
-    if (ray_trace_wave(w, st, max_iters, v, slot, wave_tame, origin))
+__device__ __forceinline__ void finish_record(const WorldView& w, const RayState& st, bool hit, const int32_t v[3],
+                                              uint32_t slot, float& t, int4& rec) {
+    if (hit)
         ray_hit_record(w, st, v, slot, t, rec);
     else
         ray_miss_record(st, t, rec);
@@ -97,7 +94,7 @@ constexpr uint32_t kGridThreads = 64;
 // most per wave and its first rows (sky) the least, so the reverse order leaves cheap
 // waves for the tail: 0.118 against 0.139 ms for the 1920x1080 primary rays.  A random
 // block order (0.145 ms) loses the L2 reuse between neighbouring tiles.
-template <bool COUNT>
+template <bool COUNT, bool GROUPS>
 __global__ __launch_bounds__(kGridThreads) void cast_grid_kernel(WorldView w, RaysIn r, HitsOut h, uint32_t max_iters,
                                                                  vrt_cast_counters* ctr, uint32_t reverse) {
     uint32_t blk = reverse ? gridDim.x - 1u - blockIdx.x : blockIdx.x;
@@ -108,8 +105,10 @@ __global__ __launch_bounds__(kGridThreads) void cast_grid_kernel(WorldView w, Ra
     int4 rec = make_int4(0, 0, 0, 0);
     if (valid) {
         ray_setup(st, r.ox[i], r.oy[i], r.oz[i], r.dx[i], r.dy[i], r.dz[i], r.W[0], r.W[1], r.W[2]);
-        // the fast loop when every ray of the wave is tame, else the exact one
-        trace_full(w, st, max_iters, __all(ray_is_tame(st)), origin_kind(r.W[0], r.W[1], r.W[2]), t, rec);
+        int32_t v[3];
+        uint32_t slot = 0;
+        const bool hit = ray_trace_wave<GROUPS>(w, st, max_iters, v, slot);
+        finish_record(w, st, hit, v, slot, t, rec);
         store_result(h, i, st, t, rec);
     }
     if constexpr (COUNT) {
@@ -143,15 +142,7 @@ struct SurvivorState {
     float2* __restrict__ b;         // per ray: side distances y, z
 };
 
-__device__ __forceinline__ void finish_record(const WorldView& w, const RayState& st, bool hit, const int32_t v[3],
-                                              uint32_t slot, float& t, int4& rec) {
-    if (hit)
-        ray_hit_record(w, st, v, slot, t, rec);
-    else
-        ray_miss_record(st, t, rec);
-}
-
-template <bool COUNT>
+template <bool COUNT, bool GROUPS>
 __global__ __launch_bounds__(kGridThreads) void cast_pass1_kernel(WorldView w, RaysIn r, HitsOut h, uint32_t cap,
                                                                   vrt_cast_counters* ctr, uint32_t reverse,
                                                                   SurvivorState q) {
@@ -164,7 +155,7 @@ __global__ __launch_bounds__(kGridThreads) void cast_pass1_kernel(WorldView w, R
         ray_setup(st, r.ox[i], r.oy[i], r.oz[i], r.dx[i], r.dy[i], r.dz[i], r.W[0], r.W[1], r.W[2]);
         int32_t v[3];
         uint32_t slot = 0;
-        hit = ray_trace_wave(w, st, cap, v, slot, __all(ray_is_tame(st)), origin_kind(r.W[0], r.W[1], r.W[2]));
+        hit = ray_trace_wave<GROUPS>(w, st, cap, v, slot);
         survivor = !hit && st.iters == cap;
         if (survivor) {
             q.a[i] = make_float4(st.cur[0], st.cur[1], st.cur[2], st.side[0]);
@@ -207,7 +198,7 @@ __device__ __forceinline__ uint32_t select_bit(uint64_t m, uint32_t k) {
 // pass-1 waves, counted in ray order.  Rounds are ngroups waves apart, so every group's
 // first round is dispatched before any second round; a round past the group's survivors
 // exits after the 64 ballot loads.
-template <bool COUNT>
+template <bool COUNT, bool GROUPS>
 __global__ __launch_bounds__(kGridThreads) void cast_pass2_kernel(WorldView w, RaysIn r, HitsOut h, uint32_t cap,
                                                                   uint32_t max_iters, vrt_cast_counters* ctr,
                                                                   SurvivorState q, uint32_t nblocks,
@@ -253,8 +244,7 @@ __global__ __launch_bounds__(kGridThreads) void cast_pass2_kernel(WorldView w, R
             st.iters = cap;
             int32_t v[3];
             uint32_t slot = 0;
-            const bool hit = ray_trace_wave(w, st, max_iters, v, slot, __all(ray_is_tame(st)),
-                                            origin_kind(r.W[0], r.W[1], r.W[2]), cap);
+            const bool hit = ray_trace_wave<GROUPS>(w, st, max_iters, v, slot, cap);
             float t;
             int4 rec;
             finish_record(w, st, hit, v, slot, t, rec);
@@ -356,7 +346,7 @@ __global__ __launch_bounds__(256) void cast_persistent_kernel(WorldView w, RaysI
             }
             if (!running && pf != ~0u) {
                 idx = pf;
-                ray_setup(st, po[0], po[1], po[2], pd[0], pd[1], pd[2], r.W[0], r.W[1], r.W[2]);
+                ray_setup_exact(st, po[0], po[1], po[2], pd[0], pd[1], pd[2], r.W[0], r.W[1], r.W[2]);
                 running = true;
                 hit = false;
                 pf = ~0u;
@@ -463,6 +453,15 @@ static int survivor_state(int dev, hipStream_t s, uint32_t n, SurvivorState* q) 
 // 0.448 ms).
 constexpr uint32_t kDefaultPassCap = 32;
 
+// Whether a cast reads the group table first (ray_trace_fast): where the step table no longer fits an
+// XCD's 4 MiB L2, and there are enough rays to be bound by the requests to it.  2 M rays without
+// order in the 2048^3 world of 587 spheres (a table of 4.8 MB): compact 497 -> 376 us, grid
+// 484 -> 421; its 1920x1080 primary rays 63.5 -> 64.4, 300 k rays 109 -> 104, 100 k 96 -> 105.  In
+// the 1024^3 terrain (0.7 MB) 2 M such rays gain 7% and 0.25 M lose 18%; in 512^3 both lose 14%.
+static bool cast_by_groups(const WorldView& w, uint32_t n) {
+    return (uint64_t)w.step_n * 16 > ((uint64_t)4 << 20) && n >= (1u << 18);
+}
+
 // Option checks that do not depend on the ray count, so a call is rejected or
 // accepted the same way whatever n is (n = 0 included).
 int check_cast_opts(const vrt_cast_opts& o) {
@@ -485,6 +484,7 @@ int launch_cast(const vrt_world* world, const RaysIn& r, const HitsOut& h, uint3
     const uint32_t cap = o.pass_cap ? o.pass_cap : kDefaultPassCap;
     // a first pass as long as the cast is the whole cast
     if (sched == VRT_SCHED_COMPACT && cap >= max_iters) sched = VRT_SCHED_GRID;
+    const bool groups = cast_by_groups(w, r.n);
     if (sched == VRT_SCHED_COMPACT) {
         SurvivorState q;
         int rc;
@@ -495,28 +495,23 @@ int launch_cast(const vrt_world* world, const RaysIn& r, const HitsOut& h, uint3
         // pass 2: 64 rounds per group of 64 ray blocks (a round past a group's survivors exits)
         const uint32_t ngroups = (blocks + kCompactGroup - 1) / kCompactGroup;
         const uint32_t waves2 = ngroups * 64u;
-        if (o.counters)
-            cast_pass1_kernel<true><<<blocks, kGridThreads, 0, s>>>(w, r, h, cap, o.counters, rev, q);
-        else
-            cast_pass1_kernel<false><<<blocks, kGridThreads, 0, s>>>(w, r, h, cap, nullptr, rev, q);
+        auto* pass1 = o.counters ? (groups ? cast_pass1_kernel<true, true> : cast_pass1_kernel<true, false>)
+                                 : (groups ? cast_pass1_kernel<false, true> : cast_pass1_kernel<false, false>);
+        pass1<<<blocks, kGridThreads, 0, s>>>(w, r, h, cap, o.counters, rev, q);
         // pass 2 reads the ballots pass 1 writes: no pass 2 after a failed pass 1
         VRT_HIP(hipGetLastError());
-        if (o.counters)
-            cast_pass2_kernel<true><<<waves2, kGridThreads, 0, s>>>(w, r, h, cap, max_iters, o.counters, q, blocks,
-                                                                   ngroups);
-        else
-            cast_pass2_kernel<false><<<waves2, kGridThreads, 0, s>>>(w, r, h, cap, max_iters, nullptr, q, blocks,
-                                                                    ngroups);
+        auto* pass2 = o.counters ? (groups ? cast_pass2_kernel<true, true> : cast_pass2_kernel<true, false>)
+                                 : (groups ? cast_pass2_kernel<false, true> : cast_pass2_kernel<false, false>);
+        pass2<<<waves2, kGridThreads, 0, s>>>(w, r, h, cap, max_iters, o.counters, q, blocks, ngroups);
         VRT_HIP(hipGetLastError());
         return VRT_OK;
     }
     if (sched == VRT_SCHED_GRID) {
         uint32_t blocks = (uint32_t)(((uint64_t)r.n + kGridThreads - 1) / kGridThreads);
         uint32_t rev = o.order == VRT_ORDER_REVERSE ? 1u : 0u;
-        if (o.counters)
-            cast_grid_kernel<true><<<blocks, kGridThreads, 0, s>>>(w, r, h, max_iters, o.counters, rev);
-        else
-            cast_grid_kernel<false><<<blocks, kGridThreads, 0, s>>>(w, r, h, max_iters, nullptr, rev);
+        auto* grid = o.counters ? (groups ? cast_grid_kernel<true, true> : cast_grid_kernel<true, false>)
+                                : (groups ? cast_grid_kernel<false, true> : cast_grid_kernel<false, false>);
+        grid<<<blocks, kGridThreads, 0, s>>>(w, r, h, max_iters, o.counters, rev);
         VRT_HIP(hipGetLastError());
         return VRT_OK;
     }

@@ -28,6 +28,8 @@ struct FwdViews {
     vrt_camera cam[kFwdViews];
     uint32_t block_begin[kFwdViews + 1];  // first block of 64 pixels of each view; [nv] = all blocks
     uint32_t pixel_base[kFwdViews];       // first output pixel of each view
+    tile_map tiles[kFwdViews];
+    float inv_w[kFwdViews], inv_h[kFwdViews];
     uint32_t nv;
 };
 
@@ -47,21 +49,15 @@ __global__ __launch_bounds__(64) void render_fwd_kernel(WorldView w, FwdViews vi
     const uint32_t i = views.pixel_base[k] + li;                          // output pixel
     RayState st;
     int32_t v[3] = {0, 0, 0};
-    bool tame = true;
     if (valid) {
         uint32_t px, py;
-        tile_pixel(li, cam.width, cam.tile_w, cam.tile_h, px, py);
+        tile_pixel(li, views.tiles[k], px, py);
         float d[3];
-        camera_ray(cam.forward, cam.right, cam.up, 1.0f / (float)cam.width, 1.0f / (float)cam.height, px, py, d);
+        camera_ray(cam.forward, cam.right, cam.up, views.inv_w[k], views.inv_h[k], px, py, d);
         ray_setup(st, cam.eye[0], cam.eye[1], cam.eye[2], d[0], d[1], d[2], cam.world_origin[0], cam.world_origin[1],
                   cam.world_origin[2]);
-        tame = ray_is_tame(st);
-    }
-    bool wave_tame = __all(tame);
-    if (valid) {
         uint32_t slot = 0;
-        bool hit = ray_trace_wave(w, st, max_iters, v, slot, wave_tame,
-                                  origin_kind(cam.world_origin[0], cam.world_origin[1], cam.world_origin[2]));
+        bool hit = ray_trace_wave(w, st, max_iters, v, slot);
         float wgt = 0.0f;
         uint32_t gv = 0xFFFFFFFFu;
         if (hit) {
@@ -428,6 +424,9 @@ int vrt_render_fwd(const vrt_world* world, const vrt_camera* cameras, uint32_t n
                 v.cam[k] = c;
                 v.block_begin[k] = (uint32_t)blocks;
                 v.pixel_base[k] = base;
+                v.tiles[k] = make_tile_map(c.width, c.tile_w, c.tile_h);
+                v.inv_w[k] = 1.0f / (float)c.width;
+                v.inv_h[k] = 1.0f / (float)c.height;
                 uint32_t n = c.width * c.height;
                 blocks += ((uint64_t)n + 63) / 64;
                 base += n;

@@ -44,6 +44,7 @@ __device__ __forceinline__ void finish_record(const WorldView& w, const RayState
 
 struct FrameArgs {
     vrt_camera cam;
+    tile_map tiles;
     float inv_w, inv_h;
     uint32_t n;
     uint32_t max_iters;
@@ -53,7 +54,7 @@ struct FrameArgs {
 
 __device__ __forceinline__ void setup_primary(const FrameArgs& a, uint32_t i, RayState& st) {
     uint32_t px, py;
-    tile_pixel(i, a.cam.width, a.cam.tile_w, a.cam.tile_h, px, py);
+    tile_pixel(i, a.tiles, px, py);
     float d[3];
     camera_ray(a.cam.forward, a.cam.right, a.cam.up, a.inv_w, a.inv_h, px, py, d);
     ray_setup(st, a.cam.eye[0], a.cam.eye[1], a.cam.eye[2], d[0], d[1], d[2], a.cam.world_origin[0],
@@ -93,15 +94,6 @@ __device__ __forceinline__ void flush4(vrt_cast_counters* ctr, unsigned long lon
 
 // ---------------------------------------------------------------- GRID
 
-// Traces the wave's active rays, with the fast step when all of them are tame;
-// true on a hit, with v the hit voxel.
-__device__ __forceinline__ bool trace_wave(const WorldView& w, RayState& st, bool active, uint32_t max_iters,
-                                           int origin, int32_t v[3], uint32_t& slot) {
-    bool tame = __all(!active || ray_is_tame(st));
-    if (!active) return false;
-    return ray_trace_wave(w, st, max_iters, v, slot, tame, origin);
-}
-
 __device__ __forceinline__ void finish_trace(const WorldView& w, const RayState& st, bool hit, const int32_t v[3],
                                              uint32_t slot, float& t, int4& rec) {
     if (hit)
@@ -122,8 +114,7 @@ __global__ __launch_bounds__(256) void frame_grid_kernel(WorldView w, FrameArgs 
     int32_t v[3] = {0, 0, 0};
     uint32_t slot = 0;
     if (valid) setup_primary(a, i, st);
-    const int origin = origin_kind(a.cam.world_origin[0], a.cam.world_origin[1], a.cam.world_origin[2]);
-    bool hit = trace_wave(w, st, valid, a.max_iters, origin, v, slot);
+    bool hit = valid && ray_trace_wave(w, st, a.max_iters, v, slot);
     bool bounce = false;
     uint32_t info = 0;
     if (valid) {
@@ -136,7 +127,7 @@ __global__ __launch_bounds__(256) void frame_grid_kernel(WorldView w, FrameArgs 
         bounce = (info & 0xFF) != 0;
         if (bounce) setup_bounce(a, i, info, st);
     }
-    hit = trace_wave(w, st, bounce, a.max_iters, origin, v, slot);
+    hit = bounce && ray_trace_wave(w, st, a.max_iters, v, slot);
     if (valid) {
         if (bounce) {
             float t;
@@ -189,6 +180,7 @@ __global__ __launch_bounds__(256) void frame_persistent_kernel(WorldView w, Fram
                 count_ray<COUNT>(c, st, rec);
                 if ((rec.w & 0xFF) != 0) {
                     setup_bounce(a, idx, (uint32_t)rec.w, st);
+                    ray_exact_inverse(st);
                     phase = LANE_BOUNCE;
                 } else {
                     float z[3] = {0.0f, 0.0f, 0.0f};
@@ -221,6 +213,7 @@ __global__ __launch_bounds__(256) void frame_persistent_kernel(WorldView w, Fram
                 if (rank < avail) {
                     idx = pool_next + rank;
                     setup_primary(a, idx, st);
+                    ray_exact_inverse(st);
                     phase = LANE_PRIMARY;
                 }
             }
@@ -280,6 +273,7 @@ extern "C" int vrt_cast_frame(const vrt_world* world, const vrt_camera* cam, uin
         hipStream_t s = (hipStream_t)stream;
         FrameArgs a;
         a.cam = *cam;
+        a.tiles = make_tile_map(cam->width, cam->tile_w, cam->tile_h);
         a.inv_w = 1.0f / (float)cam->width;
         a.inv_h = 1.0f / (float)cam->height;
         a.n = (uint32_t)n64;

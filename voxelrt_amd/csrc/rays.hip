@@ -19,14 +19,14 @@
 
 namespace vrt {
 
-__global__ __launch_bounds__(256) void camera_rays_kernel(vrt_camera cam, float inv_w, float inv_h, uint32_t n,
+__global__ __launch_bounds__(256) void camera_rays_kernel(vrt_camera cam, tile_map tiles, float inv_w, float inv_h, uint32_t n,
                                                           float* __restrict__ ox, float* __restrict__ oy,
                                                           float* __restrict__ oz, float* __restrict__ dx,
                                                           float* __restrict__ dy, float* __restrict__ dz) {
     uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= n) return;
     uint32_t px, py;
-    tile_pixel(i, cam.width, cam.tile_w, cam.tile_h, px, py);
+    tile_pixel(i, tiles, px, py);
     float d[3];
     camera_ray(cam.forward, cam.right, cam.up, inv_w, inv_h, px, py, d);
     ox[i] = cam.eye[0];
@@ -546,7 +546,7 @@ int vrt_camera_rays(const vrt_camera* cam, vrt_ray_buffers* out, void* stream) {
         if (n64 > 0xFFFFFF00ull) return fail(VRT_ERR_INVALID_ARGUMENT, "vrt_camera_rays: too many pixels");
         uint32_t n = (uint32_t)n64;
         camera_rays_kernel<<<(n + 255) / 256, 256, 0, (hipStream_t)stream>>>(
-            *cam, 1.0f / (float)cam->width, 1.0f / (float)cam->height, n, out->ox, out->oy, out->oz, out->dx, out->dy,
+            *cam, make_tile_map(cam->width, cam->tile_w, cam->tile_h), 1.0f / (float)cam->width, 1.0f / (float)cam->height, n, out->ox, out->oy, out->oz, out->dx, out->dy,
             out->dz);
         VRT_HIP(hipGetLastError());
         return VRT_OK;

@@ -21,25 +21,9 @@
 //                  the sign of a zero, which cannot change tmin + 0.001.
 // The reported t is recomputed with the exact x86 minimum in both cases.
 //
-// A third template parameter, ORIGIN, specializes the step for the rays' integer
-// world origin W (uniform over a launch or a batch segment):
-//   ORIGIN_ANY      any W: voxel = W + floor(cur), rel = aligned voxel - W;
-//   ORIGIN_ALIGNED  W a multiple of 32 on every axis (a sector corner): the
-//                   largest cell a step aligns to is 32 voxels (mask 31), so
-//                   aligning W + f and subtracting W gives the same bits as
-//                   aligning f itself; the step skips the three subtractions;
-//   ORIGIN_ZERO     W = 0: voxel = floor(cur), so the additions go as well.
-// Every form computes the same bits as ORIGIN_ANY.
-//
-// ONE_EXIT (the fast loop): the lookup is made before the bounds test, so a step
-// leaves the loop at one place for both ends of a ray.  A lane that has left the
-// world reads whatever record its index names (an index past the records reads 0:
-// the structured buffer load checks the range) and does not descend, so it never
-// reads an occupancy mask.  The loop keeps no hit flag: ray_trace tells the exits
-// apart after the loop (by the step count, or by one lookup at any origin).  Each
-// exit and flag costs lane-mask bookkeeping on the scalar unit, which one CU's four
-// SIMDs share: the one-exit step issues 18 scalar ALU instructions and 5 branches (one of
-// them skips the sector load when no lane needs it).
+// The two are steps of the exact loop and of the persistent schedules.  Every other kernel goes
+// through ray_trace_wave, whose fast loop (below) makes the same traversal with fewer
+// instructions, at any world origin W.
 #pragma once
 
 #include <hip/hip_runtime.h>
@@ -62,6 +46,26 @@ struct RayState {
 
 enum StepResult : int { STEP_CONTINUE = 0, STEP_HIT = 1, STEP_MISS = 2 };
 
+// 1 / x by V_RCP_F32 and one Newton step on its residual (Markstein, "Computation of elementary
+// functions on the IBM RISC System/6000 processor", 1990): the correctly rounded quotient for every
+// x with 2^-100 <= |x| < 2^101 (compared with 1.0f / x over all of them on this part), in 3
+// instructions instead of the 10 of a division.  Zeros, infinities and NaN give no such value.
+__device__ __forceinline__ float reciprocal_in_range(float x) {
+    const float q = __builtin_amdgcn_rcpf(x);
+    return fmaf(fmaf(-x, q, 1.0f), q, q);
+}
+
+// 1 / d and tStart by IEEE division, for any direction.
+__device__ __forceinline__ void ray_exact_inverse(RayState& r) {
+#pragma unroll
+    for (int a = 0; a < 3; a++) {
+        r.inv[a] = 1.0f / r.d[a];
+        r.ts[a] = ((r.d[a] < 0.0f ? 0.0f : 1.0f) - r.o[a]) * r.inv[a];
+    }
+}
+
+// A ray at its origin, for ray_trace_wave: 1 / d is right for the directions of quick rays
+// (ray_is_quick) only, and ray_trace_wave divides for the others.
 __device__ __forceinline__ void ray_setup(RayState& r, float ox, float oy, float oz, float dx, float dy, float dz,
                                           int32_t wx, int32_t wy, int32_t wz) {
     r.o[0] = ox; r.o[1] = oy; r.o[2] = oz;
@@ -69,7 +73,7 @@ __device__ __forceinline__ void ray_setup(RayState& r, float ox, float oy, float
     r.W[0] = wx; r.W[1] = wy; r.W[2] = wz;
 #pragma unroll
     for (int a = 0; a < 3; a++) {
-        r.inv[a] = 1.0f / r.d[a];
+        r.inv[a] = reciprocal_in_range(r.d[a]);
         r.ts[a] = ((r.d[a] < 0.0f ? 0.0f : 1.0f) - r.o[a]) * r.inv[a];
         r.side[a] = 0.0f;
         r.cur[a] = r.o[a];
@@ -83,6 +87,13 @@ __device__ __forceinline__ void ray_setup(RayState& r, float ox, float oy, float
     // records reads 0, like this initial record
     r.rec_si = ~0u;
     r.rec[0] = r.rec[1] = r.rec[2] = r.rec[3] = 0;
+}
+
+// The same for the loops that step with ray_advance.
+__device__ __forceinline__ void ray_setup_exact(RayState& r, float ox, float oy, float oz, float dx, float dy, float dz,
+                                                int32_t wx, int32_t wy, int32_t wz) {
+    ray_setup(r, ox, oy, oz, dx, dy, dz, wx, wy, wz);
+    ray_exact_inverse(r);
 }
 
 // True when the fast step is exact for this ray (see the file comment).
@@ -177,36 +188,24 @@ __device__ __forceinline__ int32_t floor_i32_in_range(float x) {
 //     is cm = ce >> min(group bits, 1); the sector record holds ce for its mask;
 //   alignment: (v & ~cm) | (dm & cm), one bitfield insert per axis.
 // Occupancy indices slot * 8 + cell are 32-bit: worlds hold at most 2^28 slots.
-enum OriginKind : int { ORIGIN_ANY = 0, ORIGIN_ALIGNED = 1, ORIGIN_ZERO = 2 };
-
-// The specialization that a world origin allows (uniform over the caller's rays).
-__device__ __forceinline__ int origin_kind(int32_t wx, int32_t wy, int32_t wz) {
-    if ((wx | wy | wz) == 0) return ORIGIN_ZERO;
-    return ((wx | wy | wz) & 31) == 0 ? ORIGIN_ALIGNED : ORIGIN_ANY;
-}
-
-template <bool EXACT, bool CUBIC = false, int ORIGIN = ORIGIN_ANY, bool ONE_EXIT = false>
+template <bool EXACT>
 __device__ __forceinline__ bool ray_advance(const WorldView& w, RayState& r, int32_t v[3], bool& hit,
                                             uint32_t* hit_slot) {
     int32_t f[3];
 #pragma unroll
     for (int a = 0; a < 3; a++) {
         f[a] = EXACT ? floor2i(r.cur[a]) : floor_i32_in_range(r.cur[a]);
-        v[a] = ORIGIN == ORIGIN_ZERO ? f[a] : (int32_t)((uint32_t)r.W[a] + (uint32_t)f[a]);
+        v[a] = (int32_t)((uint32_t)r.W[a] + (uint32_t)f[a]);
     }
-    // GetInboundMask (:114-117); one compare when the world is a cube
-    bool inb = CUBIC ? (uint32_t)(v[0] | v[1] | v[2]) < w.size_xz
-                     : ((uint32_t)(v[0] | v[2]) < w.size_xz && (uint32_t)v[1] < w.size_y);
-    if (!ONE_EXIT) {
-        if (!inb) {
-            hit = false;
-            return false;
-        }
-        r.iters++;
-        // a per-lane count: left to itself the compiler derives it from a wave-uniform loop
-        // counter with three copies per step
-        asm volatile("" : "+v"(r.iters));
+    // GetInboundMask (:114-117)
+    if (!((uint32_t)(v[0] | v[2]) < w.size_xz && (uint32_t)v[1] < w.size_y)) {
+        hit = false;
+        return false;
     }
+    r.iters++;
+    // a per-lane count: left to itself the compiler derives it from a wave-uniform loop
+    // counter with three copies per step
+    asm volatile("" : "+v"(r.iters));
     uint32_t ux = (uint32_t)v[0], uy = (uint32_t)v[1], uz = (uint32_t)v[2];
     uint32_t si = lshl_or(uy >> 5, 2 * w.shift_xz, lshl_or(uz >> 5, w.shift_xz, ux >> 5));
     // one 16-byte load for the whole record: a descent then waits on one load (the
@@ -237,7 +236,6 @@ __device__ __forceinline__ bool ray_advance(const WorldView& w, RayState& r, int
     uint32_t nbi = insert_bits_not<0x30u>(uy << 1, insert_bits<0x0Cu>(uz >> 1, ux >> 3));
     uint64_t below = m << (nbi & 63u);
     bool descend = (int32_t)(below >> 32) < 0;
-    if (ONE_EXIT) descend = descend && inb;
     // the cell mask of a step whose 2x2x2 group is empty: 15 below a sector mask, 31
     // when that mask is 0 (from the record); 1 below a voxel mask, 3 when it is 0
     uint32_t ce = sec.w;
@@ -254,14 +252,9 @@ __device__ __forceinline__ bool ray_advance(const WorldView& w, RayState& r, int
         solid = (int32_t)((m << (nbi & 63u)) >> 32) < 0;
         ce = m == 0 ? 3u : 1u;
     }
-    // the hit test after the join: its complement is then a scalar mask operation
-    // rather than a second vector compare of the sector mask (ONE_EXIT: the only exit;
-    // the lookup count then counts the steps that go on, and ray_trace adds the hit's)
-    if (ONE_EXIT) {
-        if (!inb || solid) return false;
-        r.iters++;
-        asm volatile("" : "+v"(r.iters));
-    } else if (solid) {
+    // the hit test after the join: its complement is then a scalar mask operation rather than a
+    // second vector compare of the sector mask
+    if (solid) {
         *hit_slot = slot1 - 1;
         hit = true;
         return false;
@@ -273,13 +266,8 @@ __device__ __forceinline__ bool ray_advance(const WorldView& w, RayState& r, int
 #pragma unroll
     for (int a = 0; a < 3; a++) {
         // d < 0: v & ~cm (near corner); d >= 0: v | cm (far corner); rel = that corner - W
-        int32_t rel;
-        if (ORIGIN != ORIGIN_ANY) {
-            rel = (int32_t)bitfield_insert(~cm, (uint32_t)f[a], (uint32_t)r.dm[a]);
-        } else {
-            v[a] = (int32_t)bitfield_insert(~cm, (uint32_t)v[a], (uint32_t)r.dm[a]);
-            rel = (int32_t)((uint32_t)v[a] - (uint32_t)r.W[a]);
-        }
+        v[a] = (int32_t)bitfield_insert(~cm, (uint32_t)v[a], (uint32_t)r.dm[a]);
+        const int32_t rel = (int32_t)((uint32_t)v[a] - (uint32_t)r.W[a]);
         r.side[a] = fmaf((float)rel, r.inv[a], r.ts[a]);
     }
     float tmin;
@@ -317,79 +305,318 @@ __device__ __forceinline__ uint32_t brick_slot_at(const WorldView& w, const int3
     return sec.z + (uint32_t)__popcll(m & ((1ull << bi) - 1ull));
 }
 
-// Whether voxel v (any coordinates) is solid, with its brick slot when it is.  A
-// parked ray needs no hit flag: a hit leaves v on the solid voxel, a miss outside
-// the world, and the cap on a corner of the empty cell it was stepping over.
-__device__ __forceinline__ bool solid_voxel_at(const WorldView& w, const int32_t v[3], uint32_t& slot) {
-    uint32_t ux = (uint32_t)v[0], uy = (uint32_t)v[1], uz = (uint32_t)v[2];
-    if (!((ux | uz) < w.size_xz && uy < w.size_y)) return false;
-    uint32_t si = (ux >> 5) | (uz >> 5) << w.shift_xz | (uy >> 5) << (2 * w.shift_xz);
-    uint4 sec = w.sec[si];
-    uint64_t m = (uint64_t)sec.x | (uint64_t)sec.y << 32;
-    uint32_t bi = __builtin_amdgcn_ubfe(ux, 3, 2) | __builtin_amdgcn_ubfe(uz, 3, 2) << 2 |
-                  __builtin_amdgcn_ubfe(uy, 3, 2) << 4;
-    if (!((m >> bi) & 1ull)) return false;
-    slot = sec.z + (uint32_t)__popcll(m & ((1ull << bi) - 1ull));
-    uint32_t cell = __builtin_amdgcn_ubfe(ux, 2, 1) | __builtin_amdgcn_ubfe(uz, 2, 1) << 1 |
-                    __builtin_amdgcn_ubfe(uy, 2, 1) << 2;
-    uint32_t vi = (ux & 3u) | (uz & 3u) << 2 | (uy & 3u) << 4;
-    return (w.occ[(size_t)slot * 8u + cell] >> vi) & 1ull;
+// ---------------------------------------------------------------- the fast loop
+
+// The same traversal as ray_advance, arranged for this part's issue rates.  With several waves on a
+// SIMD a wave64 instruction issues in 2 cycles when it is one of the simple ones with vector
+// operands (f32 add, multiply and fma, and / or / xor, right shifts, adds, V_BITOP3_B32), and in 4
+// when it is another (conversions, compares, minima, bitfield inserts and extracts, left and 64-bit
+// shifts, V_OR3 and the like) or reads a scalar register.  Both kinds measured with 8 waves per
+// SIMD: 2.1-2.5 and 4.1-4.3 cycles.  A step that stays at the sector level takes 34 vector
+// instructions, 10 of them of the slow kind, and 9 scalar ones and branches (ray_advance: 47, 27
+// and 23):
+//   position     g = position + bias rounded down, bias = 2^23 + W + kStepPad: the bits of g are
+//                2^23's with the padded voxel coordinate in the mantissa, so one addition in the
+//                round-down mode replaces a floor, a conversion and an addition (three axes with
+//                both mode writes: 9.6 cycles, against 21.9), and after the cell alignment
+//                g - bias is the corner relative to W as a float, exactly, with no conversion;
+//   bounds       none: the tables have a border (vrt_internal.h) whose records stop the ray;
+//   cell mask    the record holds it per 2x2x2 group (step_record);
+//   exits        one branch, taken when some lane is in an allocated brick or outside.
+// 1920x1080 frames of the 1024^3 terrain (primary and bounce rays): 234 -> 193 us with forward
+// blocks; 24 cameras and 8 ray sets in one launch: 579 -> 501 us.  The loop is no longer bound by
+// vector issue: a wave waits for its loads (a 16-byte load of 64 lanes takes an L1 17 cycles
+// however few lanes are active or lines are read) and the launch for its longest waves.
+// It is written out because the compiler's loop spends 8 more scalar instructions and a branch per
+// step on lane masks for the exits (one wave alone: 183 against 162 ns per step; ray_advance's
+// loop 219).  Waits for the loads are inside the same statement.
+//
+// Quick and guarded rays.  The border is one sector wide, so no position may leave the world by 32
+// voxels or more before its lookup.  A position is o + t d with t the least of the three computed
+// side distances, plus 0.001.  With u = 2^-24, a side distance is off by at most 2u (|o| + 1) / |d|
+// plus a relative 2u (1 / d, the difference, the product and the fma round once each, and the
+// error of 1 / d is common to both terms).  t exceeds no side distance, so on each axis the
+// position passes the cell's far plane by at most 2u (|o| + 1) + 0.002.  It can fall behind when
+// the axis that gives the minimum is far off: by 2u (|o| + 1) |1 / d| |d'| on another axis, at
+// most 16 voxels where (|o| + 1) |1 / d| <= 2^26 and |d'| <= 2.  A ray of which this holds on every
+// axis, with 0.25 <= |d|^2 <= 4, is quick (its 1 / d and tStart are then finite).  On an axis where
+// it does not (a component nudged from zero, say), the axis must never give the minimum: the
+// distance to its next voxel plane, over |d| and less the error, exceeds every t in the world.
+// Either way the ray is guarded.  Rays that are neither take ray_advance's exact step.
+__device__ __forceinline__ bool ray_is_quick(const RayState& r) {
+    // the sum bounds each axis, and a NaN on any axis fails the test
+    float x = 0.0f;
+#pragma unroll
+    for (int a = 0; a < 3; a++) x += (fabsf(r.o[a]) + 1.0f) * fabsf(r.inv[a]);
+    const float len2 = r.d[0] * r.d[0] + r.d[1] * r.d[1] + r.d[2] * r.d[2];
+    return x <= 67108864.0f && fabsf(len2 - 2.125f) <= 1.875f;
 }
 
-// RayCast's loop (CpuRenderer.cpp:185-202): steps until a hit, a miss or
+__device__ __forceinline__ bool ray_is_guarded(const WorldView& w, const RayState& r) {
+    // t of any step in the world: the longest axis of d is at least 0.28
+    const float t_max = 8.0f * (float)max(w.size_xz, w.size_y);
+    bool ok = true;
+#pragma unroll
+    for (int a = 0; a < 3; a++) {
+        const float inv = fabsf(r.inv[a]), x = (fabsf(r.o[a]) + 1.0f) * inv;
+        const float fr = r.o[a] - floorf(r.o[a]);
+        const float dist = r.d[a] < 0.0f ? fr : 1.0f - fr;
+        ok = ok && (x <= 67108864.0f || dist * inv > t_max + x * 2.384185791015625e-7f);
+    }
+    return ok;
+}
+
+// The biased coordinates need |W| well below 2^23.
+__device__ __forceinline__ bool origin_is_guarded(const int32_t W[3]) {
+    bool ok = true;
+#pragma unroll
+    for (int a = 0; a < 3; a++) ok = ok && (uint32_t)(W[a] + (1 << 20)) <= (1u << 21);
+    return ok;
+}
+
+// cur + bias per axis, rounded down.
+__device__ __forceinline__ void biased_floor(const float cur[3], const float bias[3], uint32_t g[3]) {
+    asm("s_setreg_imm32_b32 hwreg(HW_REG_MODE, 0, 2), 2\n\t"
+        "v_add_f32 %0, %3, %6\n\t"
+        "v_add_f32 %1, %4, %7\n\t"
+        "v_add_f32 %2, %5, %8\n\t"
+        "s_setreg_imm32_b32 hwreg(HW_REG_MODE, 0, 2), 0"
+        : "=&v"(g[0]), "=&v"(g[1]), "=&v"(g[2])
+        : "v"(cur[0]), "v"(cur[1]), "v"(cur[2]), "v"(bias[0]), "v"(bias[1]), "v"(bias[2]));
+}
+
+__device__ __forceinline__ i32x4 buffer_rsrc(const void* base, uint32_t stride, uint32_t records) {
+    uint64_t a = (uint64_t)base;
+    i32x4 r;
+    r.x = (int32_t)(uint32_t)a;
+    r.y = (int32_t)(((uint32_t)(a >> 32) & 0xFFFFu) | (stride << 16));
+    r.z = (int32_t)records;
+    r.w = 0x00020000;
+    return r;
+}
+
+// The parts of the fast loop (operands: ray_trace_fast).  Fixed registers: v[48:51] the kept
+// sector record, v[52:55] temporaries, v[56:57] the kept group word.
+// The side distances of the cell mask cm and the next position.
+#define VRT_STEP_ADVANCE                                       \
+    "v_bitop3_b32 %[t0], %[cm], %[m0], %[g0] bitop3:0xca\n\t"  \
+    "v_bitop3_b32 %[t1], %[cm], %[m1], %[g1] bitop3:0xca\n\t"  \
+    "v_bitop3_b32 %[t2], %[cm], %[m2], %[g2] bitop3:0xca\n\t"  \
+    "v_sub_f32 %[t0], %[t0], %[b0]\n\t"                        \
+    "v_sub_f32 %[t1], %[t1], %[b1]\n\t"                        \
+    "v_sub_f32 %[t2], %[t2], %[b2]\n\t"                        \
+    "v_fma_f32 %[s0], %[t0], %[i0], %[ts0]\n\t"                \
+    "v_fma_f32 %[s1], %[t1], %[i1], %[ts1]\n\t"                \
+    "v_fma_f32 %[s2], %[t2], %[i2], %[ts2]\n\t"                \
+    "s_add_u32 %[it], %[it], 1\n\t"                            \
+    "v_min3_f32 %[t0], %[s0], %[s1], %[s2]\n\t"                \
+    "s_cmp_ge_u32 %[it], %[max]\n\t"                           \
+    "v_add_f32 %[t0], 0x3a83126f, %[t0]\n\t"                   \
+    "v_fma_f32 %[c0], %[t0], %[d0], %[o0]\n\t"                 \
+    "v_fma_f32 %[c1], %[t0], %[d1], %[o1]\n\t"                 \
+    "v_fma_f32 %[c2], %[t0], %[d2], %[o2]\n\t"                 \
+    "s_cbranch_scc1 vrt_done%=\n\t"
+// The biased voxel coordinates: position + bias, rounded down.
+#define VRT_STEP_FLOOR                                         \
+    "s_setreg_imm32_b32 hwreg(HW_REG_MODE, 0, 2), 2\n\t"       \
+    "v_add_f32 %[g0], %[c0], %[b0]\n\t"                        \
+    "v_add_f32 %[g1], %[c1], %[b1]\n\t"                        \
+    "v_add_f32 %[g2], %[c2], %[b2]\n\t"                        \
+    "s_setreg_imm32_b32 hwreg(HW_REG_MODE, 0, 2), 0\n\t"
+// The group word, loaded by the lanes that have entered another group, and the sector's bit of
+// it: lanes of an empty sector get its cell mask, and the rest go on with exec holding them
+// (alive holds all).
+#define VRT_STEP_GROUP                                         \
+    "v_bfe_u32 %[t0], %[g0], 7, 13\n\t"                        \
+    "v_bfe_u32 %[t1], %[g1], 7, 13\n\t"                        \
+    "v_bfe_u32 %[t2], %[g2], 7, 13\n\t"                        \
+    "v_mad_u32_u24 %[t2], %[t2], %[gz], %[t0]\n\t"             \
+    "v_mad_u32_u24 %[t1], %[t1], %[gy], %[t2]\n\t"             \
+    "v_cmp_ne_u32 vcc, %[t1], %[gi]\n\t"                       \
+    "s_and_saveexec_b64 %[alive], vcc\n\t"                     \
+    "s_cbranch_execz vrt_group%=\n\t"                          \
+    "buffer_load_dwordx2 v[56:57], %[t1], %[rgrp], 0 idxen\n\t" \
+    "v_mov_b32 %[gi], %[t1]\n"                                 \
+    "vrt_group%=:\n\t"                                         \
+    "s_mov_b64 exec, %[alive]\n\t"                             \
+    "v_lshrrev_b32 %[t2], 3, %[g2]\n\t"                        \
+    "v_lshrrev_b32 %[t0], 5, %[g0]\n\t"                        \
+    "v_lshrrev_b32 %[t1], 1, %[g1]\n\t"                        \
+    "v_bitop3_b32 %[t0], 12, %[t2], %[t0] bitop3:0xca\n\t"     \
+    "v_bitop3_b32 %[t0], 48, %[t1], %[t0] bitop3:0x35\n\t"     \
+    "v_mov_b32 %[cm], 31\n\t"                                  \
+    "s_waitcnt vmcnt(0)\n\t"                                   \
+    "v_lshlrev_b64 v[52:53], %[t0], v[56:57]\n\t"              \
+    "v_cmp_gt_i32 vcc, 0, v53\n\t"                             \
+    "s_cbranch_vccz vrt_advance%=\n\t"                         \
+    "s_mov_b64 exec, vcc\n\t"
+// The sector record, loaded by the lanes that have entered another sector (lanes: what to save
+// exec in), then the brick's mask bit (v53's sign) and the sector-level cell mask.
+#define VRT_STEP_SECTOR(lanes)                                 \
+    "v_bfe_u32 %[t0], %[g0], 5, 15\n\t"                        \
+    "v_bfe_u32 %[t1], %[g1], 5, 15\n\t"                        \
+    "v_bfe_u32 %[t2], %[g2], 5, 15\n\t"                        \
+    "v_mad_u32_u24 %[t2], %[t2], %[sz], %[t0]\n\t"             \
+    "v_mad_u32_u24 %[t1], %[t1], %[sy], %[t2]\n\t"             \
+    "v_cmp_ne_u32 vcc, %[t1], %[si]\n\t"                       \
+    "s_and_saveexec_b64 " lanes ", vcc\n\t"                    \
+    "s_cbranch_execz vrt_kept%=\n\t"                           \
+    "buffer_load_dwordx4 v[48:51], %[t1], %[rsec], 0 idxen\n\t" \
+    "v_mov_b32 %[si], %[t1]\n"                                 \
+    "vrt_kept%=:\n\t"                                          \
+    "s_mov_b64 exec, " lanes "\n\t"                            \
+    "v_lshrrev_b32 %[t2], 1, %[g2]\n\t"                        \
+    "v_lshrrev_b32 %[t0], 3, %[g0]\n\t"                        \
+    "v_lshlrev_b32 %[t1], 1, %[g1]\n\t"                        \
+    "v_bitop3_b32 %[t0], 12, %[t2], %[t0] bitop3:0xca\n\t"     \
+    "v_bitop3_b32 %[t1], 48, %[t1], %[t0] bitop3:0x35\n\t"     \
+    "v_bitop3_b32 %[t0], 16, %[g1], %[t0] bitop3:0xca\n\t"     \
+    "v_and_b32 %[t0], 26, %[t0]\n\t"                           \
+    "s_waitcnt vmcnt(0)\n\t"                                   \
+    "v_lshlrev_b64 v[52:53], %[t1], v[48:49]\n\t"              \
+    "v_cmp_gt_i32 vcc, 0, v53\n\t"                             \
+    "v_lshrrev_b32 %[t0], %[t0], v51\n\t"                      \
+    "v_bitop3_b32 %[cm], %[t0], 24, 7 bitop3:0xea\n\t"
+// Lanes vcc are in an allocated brick or outside the world (the border's base slot is negative).
+// The first look their 4x4x4 cell's mask up; those that stop (a solid voxel, or outside) note
+// the step and leave exec.
+#define VRT_STEP_BRICK                                         \
+    "s_mov_b64 exec, vcc\n\t"                                  \
+    "v_cmp_gt_i32 vcc, 0, v50\n\t"                             \
+    "s_mov_b64 %[stop], vcc\n\t"                               \
+    "s_andn2_b64 exec, exec, vcc\n\t"                          \
+    "s_cbranch_execz vrt_stop%=\n\t"                           \
+    "v_bcnt_u32_b32 %[slot], v52, 0\n\t"                       \
+    "v_bcnt_u32_b32 %[slot], v53, %[slot]\n\t"                 \
+    "v_and_b32 %[t1], 4, %[g1]\n\t"                            \
+    "v_add_u32 %[slot], v50, %[slot]\n\t"                      \
+    "v_bfe_u32 %[t0], %[g0], 2, 1\n\t"                         \
+    "v_and_or_b32 %[t1], %[t2], 2, %[t1]\n\t"                  \
+    "v_lshl_or_b32 %[t0], %[slot], 3, %[t0]\n\t"               \
+    "v_or_b32 %[t0], %[t0], %[t1]\n\t"                         \
+    "buffer_load_dwordx2 v[52:53], %[t0], %[rocc], 0 idxen\n\t" \
+    "v_add_u32 %[desc], 1, %[desc]\n\t"                        \
+    "v_lshlrev_b32 %[t2], 2, %[g2]\n\t"                        \
+    "v_lshlrev_b32 %[t1], 4, %[g1]\n\t"                        \
+    "v_bitop3_b32 %[t2], 12, %[t2], %[g0] bitop3:0xca\n\t"     \
+    "v_bitop3_b32 %[t1], 48, %[t1], %[t2] bitop3:0x35\n\t"     \
+    "v_bitop3_b32 %[t2], %[t1], 42, %[t1] bitop3:0x0c\n\t"     \
+    "s_waitcnt vmcnt(0)\n\t"                                   \
+    "v_lshlrev_b64 v[54:55], %[t1], v[52:53]\n\t"              \
+    "v_or_b32 %[t0], v52, v53\n\t"                             \
+    "v_lshrrev_b64 v[52:53], %[t2], v[52:53]\n\t"              \
+    "v_cmp_gt_i32 vcc, 0, v55\n\t"                             \
+    "v_and_b32 %[t1], 0x330033, v52\n\t"                       \
+    "s_or_b64 %[stop], %[stop], vcc\n\t"                       \
+    "v_sub_u32 %[t0], 1, %[t0] clamp\n\t"                      \
+    "v_sub_u32 %[t1], 1, %[t1] clamp\n\t"                      \
+    "v_lshl_or_b32 %[cm], %[t0], 1, %[t1]\n"                   \
+    "vrt_stop%=:\n\t"                                          \
+    "s_mov_b64 exec, %[stop]\n\t"                              \
+    "v_mov_b32 %[iters], %[it]\n\t"                            \
+    "s_andn2_b64 exec, %[alive], %[stop]\n\t"                  \
+    "s_cbranch_execnz vrt_advance%=\n"
+
+// The fast loop, for quick or guarded rays.
+// GROUPS: a group word first says whether the sector is empty.  It spares a step in an empty
+// sector the record (the word serves up to four sectors of a ray), for a second load that waits on
+// the first in the others.
+template <bool GROUPS>
+__device__ __forceinline__ bool ray_trace_fast(const WorldView& w, RayState& r, uint32_t max_iters, int32_t v[3],
+                                               uint32_t& slot, uint32_t first) {
+    float bias[3];
+#pragma unroll
+    for (int a = 0; a < 3; a++) bias[a] = 8388608.0f + (float)(r.W[a] + kStepPad);
+    uint32_t g[3];
+    biased_floor(r.cur, bias, g);
+    if (first == 0) {
+        // a ray that starts outside the world misses at once; every other stays within the border
+        uint32_t u[3];
+#pragma unroll
+        for (int a = 0; a < 3; a++) u[a] = g[a] - (0x4B000000u + (uint32_t)kStepPad);
+        if (!((u[0] | u[2]) < w.size_xz && u[1] < w.size_y)) return false;
+    }
+    const i32x4 rsec = buffer_rsrc(w.steps, 16, w.step_n);
+    // slot + 1 is what a step computes: the base is one slot (8 masks) early
+    const i32x4 rocc = buffer_rsrc(w.occ - 8, 8, w.occ_n + 8u);
+    uint32_t iters = max_iters, si = ~0u, slot1 = 0, base, it = first;
+    uint32_t cm, t0, t1, t2;
+    uint64_t save, alive, stop;
+#define VRT_STEP_OPERANDS                                                                                            \
+        [c0] "+&v"(r.cur[0]), [c1] "+&v"(r.cur[1]), [c2] "+&v"(r.cur[2]), [s0] "+&v"(r.side[0]), [s1] "+&v"(r.side[1]),   \
+        [s2] "+&v"(r.side[2]), [iters] "+&v"(iters), [si] "+&v"(si), [slot] "+&v"(slot1), [desc] "+&v"(r.descents),       \
+        [it] "+&s"(it), [g0] "+&v"(g[0]), [g1] "+&v"(g[1]), [g2] "+&v"(g[2]), [cm] "=&v"(cm), [t0] "=&v"(t0),               \
+        [t1] "=&v"(t1), [t2] "=&v"(t2), [base] "=&v"(base), [save] "=&s"(save), [alive] "=&s"(alive), [stop] "=&s"(stop)
+#define VRT_STEP_INPUTS                                                                                              \
+        [o0] "v"(r.o[0]), [o1] "v"(r.o[1]), [o2] "v"(r.o[2]), [d0] "v"(r.d[0]), [d1] "v"(r.d[1]), [d2] "v"(r.d[2]),  \
+        [i0] "v"(r.inv[0]), [i1] "v"(r.inv[1]), [i2] "v"(r.inv[2]), [ts0] "v"(r.ts[0]), [ts1] "v"(r.ts[1]),          \
+        [ts2] "v"(r.ts[2]), [m0] "v"(r.dm[0]), [m1] "v"(r.dm[1]), [m2] "v"(r.dm[2]), [b0] "v"(bias[0]),              \
+        [b1] "v"(bias[1]), [b2] "v"(bias[2]), [max] "s"(max_iters), [sz] "s"(w.step_z), [sy] "s"(w.step_y),          \
+        [rsec] "s"(rsec), [rocc] "s"(rocc)
+    if constexpr (GROUPS) {
+        const i32x4 rgrp = buffer_rsrc(w.sgroups, 8, w.group_n);
+        uint32_t gi = ~0u;
+        uint64_t lanes;
+        asm volatile("s_mov_b64 %[save], exec\n\t"
+                     "s_branch vrt_look%=\n"
+                     "vrt_back%=:\n\t"
+                     "s_mov_b64 exec, %[alive]\n"
+                     "vrt_advance%=:\n\t" VRT_STEP_ADVANCE
+                     VRT_STEP_FLOOR "vrt_look%=:\n\t" VRT_STEP_GROUP VRT_STEP_SECTOR("%[lanes]")
+                     "s_cbranch_vccz vrt_back%=\n\t" VRT_STEP_BRICK
+                     "vrt_done%=:\n\t"
+                     "s_mov_b64 exec, %[save]\n\t"
+                     "v_mov_b32 %[base], v50"
+                     : VRT_STEP_OPERANDS, [gi] "+&v"(gi), [lanes] "=&s"(lanes)
+                     : VRT_STEP_INPUTS, [gz] "s"(w.group_z), [gy] "s"(w.group_y), [rgrp] "s"(rgrp)
+                     : "v48", "v49", "v50", "v51", "v52", "v53", "v54", "v55", "v56", "v57", "vcc", "scc");
+    } else {
+        asm volatile("s_mov_b64 %[save], exec\n\t"
+                     "s_branch vrt_look%=\n"
+                     "vrt_advance%=:\n\t" VRT_STEP_ADVANCE
+                     VRT_STEP_FLOOR "vrt_look%=:\n\t" VRT_STEP_SECTOR("%[alive]")
+                     "s_cbranch_vccz vrt_advance%=\n\t" VRT_STEP_BRICK
+                     "vrt_done%=:\n\t"
+                     "s_mov_b64 exec, %[save]\n\t"
+                     "v_mov_b32 %[base], v50"
+                     : VRT_STEP_OPERANDS
+                     : VRT_STEP_INPUTS
+                     : "v48", "v49", "v50", "v51", "v52", "v53", "v54", "v55", "vcc", "scc");
+    }
+#undef VRT_STEP_OPERANDS
+#undef VRT_STEP_INPUTS
+    const bool hit = iters < max_iters && (int32_t)base >= 0;
+    v[0] = (int32_t)(g[0] & 0x7FFFFFu) - kStepPad;
+    v[1] = (int32_t)(g[1] & 0x7FFFFFu) - kStepPad;
+    v[2] = (int32_t)(g[2] & 0x7FFFFFu) - kStepPad;
+    slot = slot1 - 1u;
+    r.iters = iters + (hit ? 1u : 0u);
+    return hit;
+}
+
+// RayCast's loop (CpuRenderer.cpp:185-202) in the exact form: steps until a hit, a miss or
 // max_iters steps; true on a hit, with v the hit voxel and slot its brick slot.
 // first: the steps the ray has already made (r.iters), for a ray resumed from a
 // saved position and side distances; the loop then makes at most max_iters - first.
-template <bool EXACT, bool CUBIC = false, int ORIGIN = ORIGIN_ANY>
-__device__ __forceinline__ bool ray_trace(const WorldView& w, RayState& r, uint32_t max_iters, int32_t v[3],
-                                          uint32_t& slot, uint32_t first = 0) {
+__device__ __forceinline__ bool ray_trace_exact(const WorldView& w, RayState& r, uint32_t max_iters, int32_t v[3],
+                                                uint32_t& slot, uint32_t first) {
     bool hit = false;
-    if (EXACT) {
-        for (uint32_t it = first; it < max_iters; it++)
-            if (!ray_advance<EXACT, CUBIC, ORIGIN>(w, r, v, hit, &slot)) break;
-        return hit;
-    }
-    // The fast loop has one exit and no hit flag (see ONE_EXIT above): a hit leaves v on
-    // the solid voxel, a miss outside the world, and the cap on a voxel of the empty cell
-    // it was stepping over (every entry point rejects a cap of 0, so v is set by at least
-    // one step); r.iters counts the steps that went on, max_iters only after the cap.
-    uint32_t unused;
     for (uint32_t it = first; it < max_iters; it++)
-        if (!ray_advance<EXACT, CUBIC, ORIGIN, true>(w, r, v, hit, &unused)) break;
-    if (ORIGIN == ORIGIN_ANY) {
-        // here the step overwrites v with the cell corner, and a test of the step count
-        // and v costs the loop 7 VALU instructions in exit copies: look the voxel up
-        bool h = solid_voxel_at(w, v, slot);
-        r.iters += h ? 1u : 0u;
-        return h;
-    }
-    // a hit is a ray stopped inside the world before the cap
-    uint32_t steps = r.iters;
-    bool h = steps < max_iters && (CUBIC ? (uint32_t)(v[0] | v[1] | v[2]) < w.size_xz
-                                         : ((uint32_t)(v[0] | v[2]) < w.size_xz && (uint32_t)v[1] < w.size_y));
-    if (h) slot = brick_slot_at(w, v);
-    r.iters = steps + (h ? 1u : 0u);
-    return h;
+        if (!ray_advance<true>(w, r, v, hit, &slot)) break;
+    return hit;
 }
 
-template <bool CUBIC>
-__device__ __forceinline__ bool ray_trace_tame(const WorldView& w, RayState& r, uint32_t max_iters, int32_t v[3],
-                                               uint32_t& slot, int origin, uint32_t first) {
-    if (origin == ORIGIN_ZERO) return ray_trace<false, CUBIC, ORIGIN_ZERO>(w, r, max_iters, v, slot, first);
-    if (origin == ORIGIN_ALIGNED) return ray_trace<false, CUBIC, ORIGIN_ALIGNED>(w, r, max_iters, v, slot, first);
-    return ray_trace<false, CUBIC>(w, r, max_iters, v, slot, first);
-}
-
-// ray_trace with the step picked per wave: the fast step when every ray of the
-// wave is tame (wave_tame), with the single-compare bounds test in cubic worlds
-// and specialized for the rays' world origin (origin: an OriginKind, uniform over
-// the wave).
+// The cast of a wave's rays (set up by ray_setup): the fast loop when it is exact for all of them.
+template <bool GROUPS = false>
 __device__ __forceinline__ bool ray_trace_wave(const WorldView& w, RayState& r, uint32_t max_iters, int32_t v[3],
-                                               uint32_t& slot, bool wave_tame, int origin = ORIGIN_ANY,
-                                               uint32_t first = 0) {
-    if (!wave_tame) return ray_trace<true>(w, r, max_iters, v, slot, first);
-    if (w.size_y == w.size_xz) return ray_trace_tame<true>(w, r, max_iters, v, slot, origin, first);
-    return ray_trace_tame<false>(w, r, max_iters, v, slot, origin, first);
+                                               uint32_t& slot, uint32_t first = 0) {
+    const bool near = origin_is_guarded(r.W);  // uniform
+    if (!(near && __all(ray_is_quick(r)))) {
+        ray_exact_inverse(r);
+        if (!(near && __all(ray_is_tame(r) && ray_is_guarded(w, r))))
+            return ray_trace_exact(w, r, max_iters, v, slot, first);
+    }
+    return ray_trace_fast<GROUPS>(w, r, max_iters, v, slot, first);
 }
 
 // Hit record fields (vrt_hit in vrt.h) of a finished ray.

@@ -84,9 +84,42 @@ inline uint4 sector_record(uint64_t mask, uint32_t base) {
     return make_uint4((uint32_t)mask, (uint32_t)(mask >> 32), base, mask ? 15u : 31u);
 }
 
+// What the fast step reads (ray_trace_fast): two tables over the world and a border around it, so a
+// step that leaves the world lands in the border and needs no bounds test.  Their indices come
+// from padded coordinates, the voxel's plus kStepPad (one group of 4x4x4 sectors) on each axis.
+constexpr int32_t kStepPad = 128;
+// The group table: per group of 4x4x4 sectors a u64, bit x | z << 2 | y << 4 set when that sector
+// has a brick or lies outside the world.  Group (X, Y, Z) of the padded coordinates (>> 7) is word
+// X + Z * group_z + Y * group_y.
+// The step table: per sector and for the border of one sector around the world a 16-byte record.
+// Sector (X, Y, Z) of the padded coordinates (>> 5; the world's first is 4, the border's 3) is
+// record X + Z * step_z + Y * step_y; the records before the border's first are never read.
+//   x, y  allocation mask; all ones in the border (the step's brick test then succeeds)
+//   z     base slot; all ones in the border (base slots are below 2^28)
+//   w     per 2x2x2 group of bricks (gx, gz, gy = bit 4 of x, z, y) the cell mask of a step that
+//         stays at the sector level: bits 3..4 of w >> (2 gx + 8 gz + 16 gy) are bits 3..4 of that
+//         mask, whose bits 0..2 are always set: 7 when the group holds a brick, 15 when it is
+//         empty, 31 when the sector is
+__host__ __device__ inline uint4 step_record(uint64_t mask, uint32_t base) {
+    uint32_t codes = 0;
+    for (uint32_t g = 0; g < 8; g++) {
+        const uint32_t gx = g & 1u, gz = (g >> 1) & 1u, gy = g >> 2;
+        const uint64_t group = (uint64_t)0x00330033u << (2 * gx + 8 * gz + 32 * gy);
+        const uint32_t code = mask == 0 ? 3u : ((mask & group) == 0 ? 1u : 0u);
+        codes |= code << (3 + 2 * gx + 8 * gz + 16 * gy);
+    }
+    return make_uint4((uint32_t)mask, (uint32_t)(mask >> 32), base, codes);
+}
+inline __host__ __device__ uint4 step_border_record() { return make_uint4(~0u, ~0u, ~0u, 0u); }
+
 struct WorldView {
     const uint4* __restrict__ sec;       // [nsec]
-    const uint64_t* __restrict__ occ;    // [slots * 8]
+    const uint4* __restrict__ steps;     // [step_n] the step table
+    const uint64_t* __restrict__ sgroups;  // [group_n] the group table
+    uint32_t step_z, step_y, step_n;     // their strides and sizes in records
+    uint32_t group_z, group_y, group_n;
+    const uint64_t* __restrict__ occ;    // [occ_n], slots * 8
+    uint32_t occ_n;
     const uint8_t* __restrict__ vox;     // [slots * 512]
     uint32_t size_xz, size_y;            // voxel extents
     uint32_t shift_xz, shift_y;          // log2 sector grid extents
@@ -115,6 +148,8 @@ struct vrt_world {
     uint32_t shift_xz = 0, shift_y = 0;
     uint32_t nsec = 0;
     uint4* d_sec = nullptr;           // packed sector records (mask, base slot)
+    uint4* d_steps = nullptr;         // the step table
+    uint64_t* d_sgroups = nullptr;    // the group table
     uint64_t* d_occ = nullptr;
     uint8_t* d_vox = nullptr;
     uint64_t* d_palette = nullptr;
@@ -150,10 +185,34 @@ struct vrt_world {
     // totals since creation
     uint64_t upload_bytes = 0, upload_brick_bytes = 0, moved_bricks = 0;
 
+    uint32_t step_z() const { return (1u << shift_xz) + 2u; }
+    uint32_t step_y() const { return step_z() * step_z(); }
+    uint32_t step_first() const { return 3u + 3u * step_z() + 3u * step_y(); }
+    uint32_t step_n() const { return step_first() + step_y() * ((1u << shift_y) + 2u); }
+    uint32_t group_z() const { return (1u << gshift_xz) + 2u; }
+    uint32_t group_y() const { return group_z() * group_z(); }
+    uint32_t group_n() const { return group_y() * ((1u << gshift_y) + 2u); }
+    // the bits of a group word past the end of a world of fewer than 4 sectors on an axis
+    uint64_t group_outside() const {
+        uint64_t m = 0;
+        for (uint32_t b = 0; b < 64; b++)
+            if ((b & 3u) >> shift_xz || ((b >> 2) & 3u) >> shift_xz || (b >> 4) >> shift_y) m |= 1ull << b;
+        return m;
+    }
+
     vrt::WorldView view() const {
         vrt::WorldView v;
         v.sec = d_sec;
+        v.steps = d_steps;
+        v.step_z = step_z();
+        v.step_y = step_y();
+        v.step_n = step_n();
+        v.sgroups = d_sgroups;
+        v.group_z = group_z();
+        v.group_y = group_y();
+        v.group_n = group_n();
         v.occ = d_occ;
+        v.occ_n = slot_cap * 8u;
         v.vox = d_vox;
         v.size_xz = 1u << log2_xz;
         v.size_y = 1u << log2_y;

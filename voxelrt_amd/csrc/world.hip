@@ -176,17 +176,53 @@ __global__ __launch_bounds__(256) void sync_place_kernel(uint8_t* __restrict__ v
     for (int j = 0; j < 4; j++) d4[j] = s4[j];
 }
 
-// Records of the synced sectors (indices unique) and the sector-of-sectors words they changed.
-__global__ __launch_bounds__(256) void sync_records_kernel(uint4* __restrict__ sec, const uint4* __restrict__ rec,
+// The step and group tables of an empty world: border records around records of empty sectors.
+__global__ __launch_bounds__(256) void step_tables_init_kernel(uint4* __restrict__ steps, uint32_t step_z,
+                                                               uint32_t step_y, uint32_t first, uint32_t step_n,
+                                                               uint64_t* __restrict__ groups, uint32_t group_z,
+                                                               uint32_t group_y, uint32_t group_n, uint64_t outside) {
+    uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
+    if (i < step_n) {
+        const uint32_t k = i < first ? 0u : i - first, ny = (step_n - first) / step_y;
+        const uint32_t y = k / step_y, z = k % step_y / step_z, x = k % step_z;
+        const bool border = x == 0 || x == step_z - 1 || z == 0 || z == step_z - 1 || y == 0 || y == ny - 1;
+        steps[i] = border ? step_border_record() : step_record(0, 0);
+    }
+    if (i < group_n) {
+        const uint32_t y = i / group_y, z = i % group_y / group_z, x = i % group_z;
+        const bool border =
+            x == 0 || x == group_z - 1 || z == 0 || z == group_z - 1 || y == 0 || y == group_n / group_y - 1;
+        groups[i] = border ? ~0ull : outside;
+    }
+}
+
+// Records of the synced sectors (indices unique) and the sector-of-sectors words they changed, also
+// in the fast step's tables.
+struct StepTables {
+    uint4* steps;
+    uint64_t* groups;
+    uint32_t shift_xz, gshift_xz, step_z, step_y, group_z, group_y;
+    uint64_t outside;  // bits of a group word outside the world
+};
+__global__ __launch_bounds__(256) void sync_records_kernel(uint4* __restrict__ sec, StepTables st,
+                                                           const uint4* __restrict__ rec,
                                                            const uint32_t* __restrict__ rec_idx, uint32_t nrec,
                                                            uint64_t* __restrict__ groups,
                                                            const uint64_t* __restrict__ gval,
                                                            const uint32_t* __restrict__ gidx, uint32_t ngrp) {
     uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < nrec)
-        sec[rec_idx[i]] = rec[i];
-    else if (i - nrec < ngrp)
-        groups[gidx[i - nrec]] = gval[i - nrec];
+    if (i < nrec) {
+        const uint32_t s = rec_idx[i], n1 = (1u << st.shift_xz) - 1u;
+        const uint4 r = rec[i];
+        sec[s] = r;
+        const uint32_t X = (s & n1) + 4u, Z = ((s >> st.shift_xz) & n1) + 4u, Y = (s >> (2 * st.shift_xz)) + 4u;
+        st.steps[X + Z * st.step_z + Y * st.step_y] = step_record((uint64_t)r.x | (uint64_t)r.y << 32, r.z);
+    } else if (i - nrec < ngrp) {
+        const uint32_t g = gidx[i - nrec], n1 = (1u << st.gshift_xz) - 1u;
+        groups[g] = gval[i - nrec];
+        const uint32_t X = (g & n1) + 1u, Z = ((g >> st.gshift_xz) & n1) + 1u, Y = (g >> (2 * st.gshift_xz)) + 1u;
+        st.groups[X + Z * st.group_z + Y * st.group_y] = gval[i - nrec] | st.outside;
+    }
 }
 
 }  // namespace vrt
@@ -228,6 +264,8 @@ static int grow_slots(vrt_world* w, uint32_t need, hipStream_t s) {
 
 static void free_world(vrt_world* w) {
     (void)hipFree(w->d_sec);
+    (void)hipFree(w->d_steps);
+    (void)hipFree(w->d_sgroups);
     (void)hipFree(w->d_occ);
     (void)hipFree(w->d_vox);
     (void)hipFree(w->d_palette);
@@ -514,6 +552,8 @@ static int world_sync(vrt_world* w, uint32_t nsec, const uint32_t* sector_idx, c
         gval.push_back(v);
     }
     const uint64_t nrec = nsec, ngrp = gidx.size();
+    const StepTables st{w->d_steps, w->d_sgroups, w->shift_xz, w->gshift_xz, w->step_z(), w->step_y(),
+                        w->group_z(), w->group_y(), w->group_outside()};
     for (uint64_t r0 = 0, g0 = 0; r0 < nrec || g0 < ngrp;) {
         uint32_t nr = (uint32_t)std::min<uint64_t>(nrec - r0, (kSyncHalf - 256) / 20);
         uint32_t ng = nr ? 0u : (uint32_t)std::min<uint64_t>(ngrp - g0, (kSyncHalf - 256) / 12);
@@ -531,7 +571,7 @@ static int world_sync(vrt_world* w, uint32_t nsec, const uint32_t* sector_idx, c
         e = hipMemcpyAsync(dp, hp, bytes, hipMemcpyHostToDevice, s);
         if (e == hipSuccess) {
             sync_records_kernel<<<(nr + ng + 255) / 256, 256, 0, s>>>(
-                w->d_sec, (const uint4*)dp, (const uint32_t*)(dp + o_idx), nr, w->d_groups,
+                w->d_sec, st, (const uint4*)dp, (const uint32_t*)(dp + o_idx), nr, w->d_groups,
                 (const uint64_t*)(dp + o_gval), (const uint32_t*)(dp + o_gidx), ng);
             e = hipGetLastError();
         }
@@ -606,6 +646,8 @@ int vrt_world_create(const vrt_world_desc* desc, void* stream, vrt_world** out) 
             if (e != hipSuccess && rc == VRT_OK) rc = hip_fail(e, what);
         };
         check(hipMalloc(&w->d_sec, (size_t)w->nsec * 16), "hipMalloc(sector records)");
+        check(hipMalloc(&w->d_steps, (size_t)w->step_n() * 16), "hipMalloc(step table)");
+        check(hipMalloc(&w->d_sgroups, (size_t)w->group_n() * 8), "hipMalloc(group table)");
         check(hipMalloc(&w->d_palette, 256 * 8), "hipMalloc(palette)");
         check(hipMalloc(&w->d_groups, w->h_groups.size() * 8), "hipMalloc(sector groups)");
         check(hipMalloc(&w->d_lut, 512 * 8), "hipMalloc(ray-cell table)");
@@ -613,6 +655,10 @@ int vrt_world_create(const vrt_world_desc* desc, void* stream, vrt_world** out) 
             std::vector<uint4> empty(w->nsec, sector_record(0, 0));
             check(hipMemcpyAsync(w->d_sec, empty.data(), (size_t)w->nsec * 16, hipMemcpyHostToDevice, s),
                   "hipMemcpyAsync(sector records)");
+            step_tables_init_kernel<<<(std::max(w->step_n(), w->group_n()) + 255) / 256, 256, 0, s>>>(
+                w->d_steps, w->step_z(), w->step_y(), w->step_first(), w->step_n(), w->d_sgroups, w->group_z(),
+                w->group_y(), w->group_n(), w->group_outside());
+            check(hipGetLastError(), "step_tables_init_kernel");
             check(hipStreamSynchronize(s), "hipStreamSynchronize(sector records)");
             check(hipMemsetAsync(w->d_palette, 0, 256 * 8, s), "hipMemsetAsync(palette)");
             check(hipMemsetAsync(w->d_groups, 0, w->h_groups.size() * 8, s), "hipMemsetAsync(sector groups)");
@@ -648,7 +694,7 @@ int vrt_world_get_info(const vrt_world* w, vrt_world_info* out) {
         out->num_sectors = w->nsec;
         out->num_bricks = w->num_bricks;
         out->slot_capacity = w->slot_cap;
-        out->device_bytes = (uint64_t)w->nsec * 16 + 256 * 8 + (uint64_t)w->slot_cap * (512 + 64) +
+        out->device_bytes = (uint64_t)w->nsec * 16 + (uint64_t)w->step_n() * 16 + (uint64_t)w->group_n() * 8 + 256 * 8 + (uint64_t)w->slot_cap * (512 + 64) +
                             (uint64_t)w->h_groups.size() * 8 + 512 * 8 + (w->d_stage ? 2 * kSyncHalf : 0) +
                             w->moves_cap;
         out->slot_high_water = w->arena.high_water();

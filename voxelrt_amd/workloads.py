@@ -9,8 +9,7 @@
     C5  512^3 terrain, 16 views of 512x512, per-voxel RGB albedo (differentiable)
 
 The C2, C4 and C5 cameras put their rays' integer world origin at the corner of the
-camera's sector (a multiple of 32 per axis: the casts' aligned-origin step); C1 and C3
-at floor(eye), the reference's choice (the general step).
+camera's sector (a multiple of 32 per axis); C1 and C3 at floor(eye), the reference's choice.
 """
 from __future__ import annotations
 
