@@ -19,6 +19,15 @@ namespace vrt {
 
 __device__ __forceinline__ bool fine_bit(uint64_t m, uint32_t idx) { return (m >> (idx & 63u)) & 1u; }
 
+// findAnyOccupiedPos (:40-52): v moved to the lowest set bit of its cell's mask, low word first.
+__device__ __forceinline__ void first_occupied(uint64_t m, int32_t v[3]) {
+    uint32_t bit = (uint32_t)m != 0 ? (uint32_t)__builtin_ctz((uint32_t)m)
+                                    : 32u + (uint32_t)__builtin_ctz((uint32_t)(m >> 32));
+    v[0] = (v[0] & ~3) | (int32_t)(bit & 3u);
+    v[1] = (v[1] & ~3) | (int32_t)((bit >> 4) & 3u);
+    v[2] = (v[2] & ~3) | (int32_t)((bit >> 2) & 3u);
+}
+
 // getStepPos (:92-131).  Returns true when v is solid (or, for a coarse step, when v
 // was moved to the first solid voxel of its non-empty 4x4x4 cell); otherwise moves v
 // to the far corner, in ray direction, of the largest empty aligned cell.
@@ -59,12 +68,7 @@ __device__ __forceinline__ bool shader_step(const ShaderView& sv, int32_t v[3], 
     }
     int32_t lod = iso * scale;
     if (coarse && lod < 4) {
-        // findAnyOccupiedPos (:40-52): lowest set bit, low word first
-        uint32_t bit = (uint32_t)m != 0 ? (uint32_t)__builtin_ctz((uint32_t)m)
-                                        : 32u + (uint32_t)__builtin_ctz((uint32_t)(m >> 32));
-        v[0] = (v[0] & ~3) | (int32_t)(bit & 3u);
-        v[1] = (v[1] & ~3) | (int32_t)((bit >> 4) & 3u);
-        v[2] = (v[2] & ~3) | (int32_t)((bit >> 2) & 3u);
+        first_occupied(m, v);
         return true;
     }
     // d < 0: v & ~cm, else v | cm (the fast loop: one bitfield insert of dm, all ones unless
@@ -77,17 +81,16 @@ __device__ __forceinline__ bool shader_step(const ShaderView& sv, int32_t v[3], 
     return false;
 }
 
-// clipRayToAABB (:133-145) against [1 - W, size - W - 1].
-__device__ __forceinline__ void clip_ray(const WorldView& w, const float o[3], const float d[3], const int32_t W[3],
-                                         float out[3]) {
+// clipRayToAABB (:133-145) against [1 - W, size - W - 1]; inv: 1 / d.
+__device__ __forceinline__ void clip_ray(const WorldView& w, const float o[3], const float d[3], const float inv[3],
+                                         const int32_t W[3], float out[3]) {
     float size[3] = {(float)w.size_xz, (float)w.size_y, (float)w.size_xz};
     float lo[3], hi[3];
 #pragma unroll
     for (int a = 0; a < 3; a++) {
-        float inv = 1.0f / d[a];
         float bmin = (float)(int32_t)(1u - (uint32_t)W[a]);
         float bmax = (size[a] - (float)W[a]) - 1.0f;
-        float t1 = (bmin - o[a]) * inv, t2 = (bmax - o[a]) * inv;
+        float t1 = (bmin - o[a]) * inv[a], t2 = (bmax - o[a]) * inv[a];
         lo[a] = fminf(t1, t2);
         hi[a] = fmaxf(t1, t2);
     }
@@ -142,37 +145,128 @@ __device__ __forceinline__ bool shader_loop(const ShaderView& sv, const float d[
     return hit;
 }
 
-// rayCast (COARSE = false, :162-204) or rayCastCoarse (COARSE = true, :206-243).  FAST
-// takes the tame loop when every ray of the wave is tame.
-template <bool COARSE, bool LUT, bool FAST = !COARSE>
+// shader_loop without the ray-cell table for quick rays (ray_is_quick of the start org, d and inv), in
+// worlds of at least 128 voxels on every axis: the cast's fast loop (traverse.h) with this method's
+// bias, its level above an empty sector (step records' bits 8..9) and rayCastCoarse's stop in a
+// non-empty cell from step 31 on.  The largest cell, 128 voxels, then lies inside the world, so
+// positions stay within the tables' border as there.  A step at the sector level takes 36 vector
+// instructions (shader_loop's about 70, with no record kept between steps): 2.07 M camera rays over
+// the 1024^3 terrain 167 -> 96 us (rayCast), 80 -> 45 us (rayCastCoarse).  slot: the hit voxel's
+// brick.
+template <bool COARSE>
+__device__ __forceinline__ bool shader_loop_fast(const WorldView& w, const float d[3], const float org[3],
+                                                 const float inv[3], const float ts[3], const int32_t W[3],
+                                                 const int32_t dm[3], uint32_t cap, int32_t v[3], float side[3],
+                                                 float cur[3], float& tmin, uint32_t& steps, uint32_t& slot) {
+    // the first step leaves the start's voxel, which may lie anywhere
+#pragma unroll
+    for (int a = 0; a < 3; a++)
+        side[a] = fmaf((float)(int32_t)((uint32_t)v[a] - (uint32_t)W[a]), inv[a], ts[a]);
+    tmin = fminf(fminf(side[0], side[1]), side[2]);
+    tmin = COARSE ? tmin + 0.001f : __uint_as_float(__float_as_uint(tmin) + 5u);
+    float bias3[3];
+#pragma unroll
+    for (int a = 0; a < 3; a++) {
+        cur[a] = fmaf(tmin, d[a], org[a]);
+        bias3[a] = 8388608.0f + (float)(W[a] + kStepPad);
+    }
+    uint32_t g[3], u[3];
+    biased_floor(cur, bias3, g);
+#pragma unroll
+    for (int a = 0; a < 3; a++) u[a] = g[a] - (0x4B000000u + (uint32_t)kStepPad);
+    steps = 0;
+    if (!((u[0] | u[2]) < w.size_xz && u[1] < w.size_y)) return false;
+    const i32x4 rsec = buffer_rsrc(w.steps, 16, w.step_n);
+    const i32x4 rocc = buffer_rsrc(w.occ - 8, 8, w.occ_n + 8u);
+    uint32_t iters = cap, si = ~0u, slot1 = 0, base, it = 0;
+    uint32_t cm, t0, t1, t2, mlo, mhi;
+    uint64_t save, alive, stop;
+#define VRT_SHADER_STEP(bias, coarse)                                                                           \
+    asm volatile("s_mov_b64 %[save], exec\n\t"                                                                  \
+                 "s_branch vrt_look%=\n"                                                                        \
+                 "vrt_advance%=:\n\t" VRT_STEP_ADVANCE("%[tm]", bias) VRT_STEP_FLOOR                            \
+                 "vrt_look%=:\n\t" VRT_STEP_SECTOR("%[alive]")                                                  \
+                 "v_lshrrev_b32 %[t0], 3, v51\n\t"                                                              \
+                 "v_and_or_b32 %[cm], %[t0], %[lod], %[cm]\n\t"                                                 \
+                 "s_cbranch_vccz vrt_advance%=\n\t" VRT_STEP_CELL coarse VRT_STEP_STOP                          \
+                 "vrt_done%=:\n\t"                                                                              \
+                 "s_mov_b64 exec, %[save]\n\t"                                                                  \
+                 "v_mov_b32 %[base], v50\n\t"                                                                   \
+                 "v_mov_b32 %[mlo], v52\n\t"                                                                    \
+                 "v_mov_b32 %[mhi], v53"                                                                        \
+                 : VRT_STEP_OUT(cur, side, g), [tm] "+&v"(tmin), [mlo] "=&v"(mlo), [mhi] "=&v"(mhi)             \
+                 : VRT_STEP_IN(org, d, inv, ts, dm, bias3, cap), [lod] "s"(0x60u)                               \
+                 : VRT_STEP_CLOBBERS)
+    if constexpr (COARSE)
+        VRT_SHADER_STEP("v_add_f32 %[tm], 0x3a83126f, %[tm]\n\t",
+                        // any voxel of the cell stops the ray once it > 30 (t0: its mask, ored)
+                        "v_cmp_ne_u32 vcc, 0, %[t0]\n\t"
+                        "s_cmp_gt_u32 %[it], 30\n\t"
+                        "s_cselect_b64 vcc, vcc, 0\n\t"
+                        "s_or_b64 %[stop], %[stop], vcc\n\t");
+    else
+        VRT_SHADER_STEP("v_add_u32 %[tm], 5, %[tm]\n\t", "");
+#undef VRT_SHADER_STEP
+    const bool hit = iters < cap && (int32_t)base >= 0;
+    steps = iters;
+    slot = slot1 - 1u;
+#pragma unroll
+    for (int a = 0; a < 3; a++) v[a] = (int32_t)(g[a] & 0x7FFFFFu) - kStepPad;
+    if (COARSE && hit) {
+        const uint64_t m = (uint64_t)mlo | (uint64_t)mhi << 32;
+        const uint32_t vi = ((uint32_t)v[0] & 3u) | ((uint32_t)v[2] & 3u) << 2 | ((uint32_t)v[1] & 3u) << 4;
+        if (!fine_bit(m, vi)) first_occupied(m, v);
+    }
+    return hit;
+}
+
+// rayCast (COARSE = false, :162-204) or rayCastCoarse (COARSE = true, :206-243).
+template <bool COARSE, bool LUT>
 __device__ __forceinline__ bool shader_trace(const ShaderView& sv, const float o[3], const float d[3],
                                              const int32_t W[3], uint32_t cap, ShaderHit& out) {
     const WorldView& w = sv.w;
     float start[3], org[3], inv[3], ts[3], side[3] = {0.0f, 0.0f, 0.0f}, cur[3] = {0.0f, 0.0f, 0.0f};
-    clip_ray(w, o, d, W, start);
     int32_t v[3], dm[3];
-    bool tame = true;
+    auto begin = [&] {
+        clip_ray(w, o, d, inv, W, start);
 #pragma unroll
-    for (int a = 0; a < 3; a++) {
-        org[a] = COARSE ? start[a] : o[a];
-        inv[a] = 1.0f / d[a];
-        ts[a] = ((d[a] < 0.0f ? 0.0f : 1.0f) - org[a]) * inv[a];
-        v[a] = (int32_t)((uint32_t)W[a] + (uint32_t)floor2i(start[a]));
-        dm[a] = d[a] < 0.0f ? 0 : -1;
-        tame = tame && fabsf(inv[a]) < INFINITY && fabsf(ts[a]) < INFINITY && fabsf(org[a]) < 1048576.0f;
-    }
-    float len2 = d[0] * d[0] + d[1] * d[1] + d[2] * d[2];
-    tame = tame && len2 >= 0.25f && len2 <= 4.0f;
-    const uint32_t oct = (d[0] < 0.0f ? 0u : 1u) + (d[1] < 0.0f ? 0u : 2u) + (d[2] < 0.0f ? 0u : 4u);
+        for (int a = 0; a < 3; a++) {
+            org[a] = COARSE ? start[a] : o[a];
+            ts[a] = ((d[a] < 0.0f ? 0.0f : 1.0f) - org[a]) * inv[a];
+            v[a] = (int32_t)((uint32_t)W[a] + (uint32_t)floor2i(start[a]));
+            dm[a] = d[a] < 0.0f ? 0 : -1;
+        }
+    };
     float tmin = 0.0f;
-    uint32_t it = 0;
-    // the fast loop by default for rayCast only: inside the renderer rayCastCoarse's short
-    // traces (cap 96, shadow and bounce rays) measured no gain from it, and its second loop
-    // copy slowed the renderer's kernel, which holds three traces; the batch kernel, which
-    // holds one, takes it for both (coarse C2 camera rays: 14.8 against 13.8 Grays/s)
-    bool hit = FAST && __all(tame)
-                   ? shader_loop<COARSE, LUT, true>(sv, d, org, inv, ts, W, dm, oct, cap, v, side, cur, tmin, it)
-                   : shader_loop<COARSE, LUT, false>(sv, d, org, inv, ts, W, dm, oct, cap, v, side, cur, tmin, it);
+    uint32_t it = 0, slot = 0;
+    bool hit, tame = true, found = false;
+    if constexpr (!LUT) {
+#pragma unroll
+        for (int a = 0; a < 3; a++) inv[a] = reciprocal_in_range(d[a]);
+        begin();
+        // uniform: the launch's world and world origin
+        const bool fits = origin_is_guarded(W) && w.size_xz >= 128 && w.size_y >= 128;
+        if (fits && __all(ray_is_quick(org, d, inv))) {
+            hit = shader_loop_fast<COARSE>(w, d, org, inv, ts, W, dm, cap, v, side, cur, tmin, it, slot);
+            found = true;
+        }
+    }
+    if (!found) {
+#pragma unroll
+        for (int a = 0; a < 3; a++) inv[a] = 1.0f / d[a];
+        begin();
+#pragma unroll
+        for (int a = 0; a < 3; a++)
+            tame = tame && fabsf(inv[a]) < INFINITY && fabsf(ts[a]) < INFINITY && fabsf(org[a]) < 1048576.0f;
+        float len2 = d[0] * d[0] + d[1] * d[1] + d[2] * d[2];
+        tame = tame && len2 >= 0.25f && len2 <= 4.0f;
+        const uint32_t oct = (d[0] < 0.0f ? 0u : 1u) + (d[1] < 0.0f ? 0u : 2u) + (d[2] < 0.0f ? 0u : 4u);
+        if (LUT && __all(tame))
+            hit = shader_loop<COARSE, LUT, true>(sv, d, org, inv, ts, W, dm, oct, cap, v, side, cur, tmin, it);
+        else
+            hit = shader_loop<COARSE, LUT, false>(sv, d, org, inv, ts, W, dm, oct, cap, v, side, cur, tmin, it);
+        if (hit) slot = brick_slot_at(w, v);
+    }
     // the record is built in locals and stored once, so the result stays in registers
     uint32_t code = 0, mat = 0;
     float t = -1.0f;
@@ -183,12 +277,6 @@ __device__ __forceinline__ bool shader_trace(const ShaderView& sv, const float o
         for (int a = 0; a < 3; a++)
             if (tmin >= side[a]) code |= (d[a] < 0.0f ? 1u : (d[a] > 0.0f ? 3u : 0u)) << (2 * a);
         uint32_t ux = (uint32_t)v[0], uy = (uint32_t)v[1], uz = (uint32_t)v[2];
-        uint32_t si = (ux >> 5) | (uz >> 5) << w.shift_xz | (uy >> 5) << (2 * w.shift_xz);
-        uint4 sec = w.sec[si];
-        uint64_t m = (uint64_t)sec.x | (uint64_t)sec.y << 32;
-        uint32_t bi = __builtin_amdgcn_ubfe(ux, 3, 2) | __builtin_amdgcn_ubfe(uz, 3, 2) << 2 |
-                      __builtin_amdgcn_ubfe(uy, 3, 2) << 4;
-        uint32_t slot = sec.z + (uint32_t)__popcll(m & ((1ull << bi) - 1ull));
         mat = w.vox[(size_t)slot * 512 + ((ux & 7u) | (uz & 7u) << 3 | (uy & 7u) << 6)];
         t = tmin;
 #pragma unroll

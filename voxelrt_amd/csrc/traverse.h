@@ -343,12 +343,12 @@ __device__ __forceinline__ uint32_t brick_slot_at(const WorldView& w, const int3
 // it does not (a component nudged from zero, say), the axis must never give the minimum: the
 // distance to its next voxel plane, over |d| and less the error, exceeds every t in the world.
 // Either way the ray is guarded.  Rays that are neither take ray_advance's exact step.
-__device__ __forceinline__ bool ray_is_quick(const RayState& r) {
+__device__ __forceinline__ bool ray_is_quick(const float o[3], const float d[3], const float inv[3]) {
     // the sum bounds each axis, and a NaN on any axis fails the test
     float x = 0.0f;
 #pragma unroll
-    for (int a = 0; a < 3; a++) x += (fabsf(r.o[a]) + 1.0f) * fabsf(r.inv[a]);
-    const float len2 = r.d[0] * r.d[0] + r.d[1] * r.d[1] + r.d[2] * r.d[2];
+    for (int a = 0; a < 3; a++) x += (fabsf(o[a]) + 1.0f) * fabsf(inv[a]);
+    const float len2 = d[0] * d[0] + d[1] * d[1] + d[2] * d[2];
     return x <= 67108864.0f && fabsf(len2 - 2.125f) <= 1.875f;
 }
 
@@ -397,8 +397,9 @@ __device__ __forceinline__ i32x4 buffer_rsrc(const void* base, uint32_t stride, 
 
 // The parts of the fast loop (operands: ray_trace_fast).  Fixed registers: v[48:51] the kept
 // sector record, v[52:55] temporaries, v[56:57] the kept group word.
-// The side distances of the cell mask cm and the next position.
-#define VRT_STEP_ADVANCE                                       \
+// The side distances of the cell mask cm and the next position; bias: what is added to the least
+// of them (in register tmin).
+#define VRT_STEP_ADVANCE(tmin, bias)                           \
     "v_bitop3_b32 %[t0], %[cm], %[m0], %[g0] bitop3:0xca\n\t"  \
     "v_bitop3_b32 %[t1], %[cm], %[m1], %[g1] bitop3:0xca\n\t"  \
     "v_bitop3_b32 %[t2], %[cm], %[m2], %[g2] bitop3:0xca\n\t"  \
@@ -409,13 +410,14 @@ __device__ __forceinline__ i32x4 buffer_rsrc(const void* base, uint32_t stride, 
     "v_fma_f32 %[s1], %[t1], %[i1], %[ts1]\n\t"                \
     "v_fma_f32 %[s2], %[t2], %[i2], %[ts2]\n\t"                \
     "s_add_u32 %[it], %[it], 1\n\t"                            \
-    "v_min3_f32 %[t0], %[s0], %[s1], %[s2]\n\t"                \
+    "v_min3_f32 " tmin ", %[s0], %[s1], %[s2]\n\t"             \
     "s_cmp_ge_u32 %[it], %[max]\n\t"                           \
-    "v_add_f32 %[t0], 0x3a83126f, %[t0]\n\t"                   \
-    "v_fma_f32 %[c0], %[t0], %[d0], %[o0]\n\t"                 \
-    "v_fma_f32 %[c1], %[t0], %[d1], %[o1]\n\t"                 \
-    "v_fma_f32 %[c2], %[t0], %[d2], %[o2]\n\t"                 \
+    bias                                                       \
+    "v_fma_f32 %[c0], " tmin ", %[d0], %[o0]\n\t"              \
+    "v_fma_f32 %[c1], " tmin ", %[d1], %[o1]\n\t"              \
+    "v_fma_f32 %[c2], " tmin ", %[d2], %[o2]\n\t"              \
     "s_cbranch_scc1 vrt_done%=\n\t"
+#define VRT_STEP_BIAS "v_add_f32 %[t0], 0x3a83126f, %[t0]\n\t" /* + 0.001 */
 // The biased voxel coordinates: position + bias, rounded down.
 #define VRT_STEP_FLOOR                                         \
     "s_setreg_imm32_b32 hwreg(HW_REG_MODE, 0, 2), 2\n\t"       \
@@ -478,9 +480,9 @@ __device__ __forceinline__ i32x4 buffer_rsrc(const void* base, uint32_t stride, 
     "v_lshrrev_b32 %[t0], %[t0], v51\n\t"                      \
     "v_bitop3_b32 %[cm], %[t0], 24, 7 bitop3:0xea\n\t"
 // Lanes vcc are in an allocated brick or outside the world (the border's base slot is negative).
-// The first look their 4x4x4 cell's mask up; those that stop (a solid voxel, or outside) note
-// the step and leave exec.
-#define VRT_STEP_BRICK                                         \
+// The first look their 4x4x4 cell's mask up (v[52:53]; slot: their brick's slot + 1), and stop at
+// a solid voxel; t1 and t2 are the voxel's shifts.
+#define VRT_STEP_CELL                                          \
     "s_mov_b64 exec, vcc\n\t"                                  \
     "v_cmp_gt_i32 vcc, 0, v50\n\t"                             \
     "s_mov_b64 %[stop], vcc\n\t"                               \
@@ -495,7 +497,6 @@ __device__ __forceinline__ i32x4 buffer_rsrc(const void* base, uint32_t stride, 
     "v_lshl_or_b32 %[t0], %[slot], 3, %[t0]\n\t"               \
     "v_or_b32 %[t0], %[t0], %[t1]\n\t"                         \
     "buffer_load_dwordx2 v[52:53], %[t0], %[rocc], 0 idxen\n\t" \
-    "v_add_u32 %[desc], 1, %[desc]\n\t"                        \
     "v_lshlrev_b32 %[t2], 2, %[g2]\n\t"                        \
     "v_lshlrev_b32 %[t1], 4, %[g1]\n\t"                        \
     "v_bitop3_b32 %[t2], 12, %[t2], %[g0] bitop3:0xca\n\t"     \
@@ -504,10 +505,13 @@ __device__ __forceinline__ i32x4 buffer_rsrc(const void* base, uint32_t stride, 
     "s_waitcnt vmcnt(0)\n\t"                                   \
     "v_lshlrev_b64 v[54:55], %[t1], v[52:53]\n\t"              \
     "v_or_b32 %[t0], v52, v53\n\t"                             \
-    "v_lshrrev_b64 v[52:53], %[t2], v[52:53]\n\t"              \
     "v_cmp_gt_i32 vcc, 0, v55\n\t"                             \
-    "v_and_b32 %[t1], 0x330033, v52\n\t"                       \
+    "v_lshrrev_b64 v[54:55], %[t2], v[52:53]\n\t"              \
     "s_or_b64 %[stop], %[stop], vcc\n\t"                       \
+    "v_and_b32 %[t1], 0x330033, v54\n\t"
+// t0: the cell's mask, ored; t1: its 2x2x2 group's.  Cell mask 3 when the first is 0, 1 when the
+// second is.  The lanes that stop note the step and leave exec.
+#define VRT_STEP_STOP                                          \
     "v_sub_u32 %[t0], 1, %[t0] clamp\n\t"                      \
     "v_sub_u32 %[t1], 1, %[t1] clamp\n\t"                      \
     "v_lshl_or_b32 %[cm], %[t0], 1, %[t1]\n"                   \
@@ -516,6 +520,21 @@ __device__ __forceinline__ i32x4 buffer_rsrc(const void* base, uint32_t stride, 
     "v_mov_b32 %[iters], %[it]\n\t"                            \
     "s_andn2_b64 exec, %[alive], %[stop]\n\t"                  \
     "s_cbranch_execnz vrt_advance%=\n"
+#define VRT_STEP_BRICK VRT_STEP_CELL "v_add_u32 %[desc], 1, %[desc]\n\t" VRT_STEP_STOP
+
+// Operands of both loops (positions c, side distances s, directions d, 1 / d i, tStart ts, origin o,
+// corner masks m, bias b, per axis).
+#define VRT_STEP_OUT(C, S, G)                                                                                   \
+    [c0] "+&v"(C[0]), [c1] "+&v"(C[1]), [c2] "+&v"(C[2]), [s0] "+&v"(S[0]), [s1] "+&v"(S[1]), [s2] "+&v"(S[2]), \
+        [g0] "+&v"(G[0]), [g1] "+&v"(G[1]), [g2] "+&v"(G[2]), [iters] "+&v"(iters), [si] "+&v"(si),             \
+        [slot] "+&v"(slot1), [it] "+&s"(it), [cm] "=&v"(cm), [t0] "=&v"(t0), [t1] "=&v"(t1), [t2] "=&v"(t2),    \
+        [base] "=&v"(base), [save] "=&s"(save), [alive] "=&s"(alive), [stop] "=&s"(stop)
+#define VRT_STEP_IN(O, D, I, T, M, B, cap)                                                                      \
+    [o0] "v"(O[0]), [o1] "v"(O[1]), [o2] "v"(O[2]), [d0] "v"(D[0]), [d1] "v"(D[1]), [d2] "v"(D[2]),             \
+        [i0] "v"(I[0]), [i1] "v"(I[1]), [i2] "v"(I[2]), [ts0] "v"(T[0]), [ts1] "v"(T[1]), [ts2] "v"(T[2]),      \
+        [m0] "v"(M[0]), [m1] "v"(M[1]), [m2] "v"(M[2]), [b0] "v"(B[0]), [b1] "v"(B[1]), [b2] "v"(B[2]),         \
+        [max] "s"(cap), [sz] "s"(w.step_z), [sy] "s"(w.step_y), [rsec] "s"(rsec), [rocc] "s"(rocc)
+#define VRT_STEP_CLOBBERS "v48", "v49", "v50", "v51", "v52", "v53", "v54", "v55", "vcc", "scc"
 
 // The fast loop, for quick or guarded rays.
 // GROUPS: a group word first says whether the sector is empty.  It spares a step in an empty
@@ -542,17 +561,6 @@ __device__ __forceinline__ bool ray_trace_fast(const WorldView& w, RayState& r, 
     uint32_t iters = max_iters, si = ~0u, slot1 = 0, base, it = first;
     uint32_t cm, t0, t1, t2;
     uint64_t save, alive, stop;
-#define VRT_STEP_OPERANDS                                                                                            \
-        [c0] "+&v"(r.cur[0]), [c1] "+&v"(r.cur[1]), [c2] "+&v"(r.cur[2]), [s0] "+&v"(r.side[0]), [s1] "+&v"(r.side[1]),   \
-        [s2] "+&v"(r.side[2]), [iters] "+&v"(iters), [si] "+&v"(si), [slot] "+&v"(slot1), [desc] "+&v"(r.descents),       \
-        [it] "+&s"(it), [g0] "+&v"(g[0]), [g1] "+&v"(g[1]), [g2] "+&v"(g[2]), [cm] "=&v"(cm), [t0] "=&v"(t0),               \
-        [t1] "=&v"(t1), [t2] "=&v"(t2), [base] "=&v"(base), [save] "=&s"(save), [alive] "=&s"(alive), [stop] "=&s"(stop)
-#define VRT_STEP_INPUTS                                                                                              \
-        [o0] "v"(r.o[0]), [o1] "v"(r.o[1]), [o2] "v"(r.o[2]), [d0] "v"(r.d[0]), [d1] "v"(r.d[1]), [d2] "v"(r.d[2]),  \
-        [i0] "v"(r.inv[0]), [i1] "v"(r.inv[1]), [i2] "v"(r.inv[2]), [ts0] "v"(r.ts[0]), [ts1] "v"(r.ts[1]),          \
-        [ts2] "v"(r.ts[2]), [m0] "v"(r.dm[0]), [m1] "v"(r.dm[1]), [m2] "v"(r.dm[2]), [b0] "v"(bias[0]),              \
-        [b1] "v"(bias[1]), [b2] "v"(bias[2]), [max] "s"(max_iters), [sz] "s"(w.step_z), [sy] "s"(w.step_y),          \
-        [rsec] "s"(rsec), [rocc] "s"(rocc)
     if constexpr (GROUPS) {
         const i32x4 rgrp = buffer_rsrc(w.sgroups, 8, w.group_n);
         uint32_t gi = ~0u;
@@ -561,30 +569,28 @@ __device__ __forceinline__ bool ray_trace_fast(const WorldView& w, RayState& r, 
                      "s_branch vrt_look%=\n"
                      "vrt_back%=:\n\t"
                      "s_mov_b64 exec, %[alive]\n"
-                     "vrt_advance%=:\n\t" VRT_STEP_ADVANCE
+                     "vrt_advance%=:\n\t" VRT_STEP_ADVANCE("%[t0]", VRT_STEP_BIAS)
                      VRT_STEP_FLOOR "vrt_look%=:\n\t" VRT_STEP_GROUP VRT_STEP_SECTOR("%[lanes]")
                      "s_cbranch_vccz vrt_back%=\n\t" VRT_STEP_BRICK
                      "vrt_done%=:\n\t"
                      "s_mov_b64 exec, %[save]\n\t"
                      "v_mov_b32 %[base], v50"
-                     : VRT_STEP_OPERANDS, [gi] "+&v"(gi), [lanes] "=&s"(lanes)
-                     : VRT_STEP_INPUTS, [gz] "s"(w.group_z), [gy] "s"(w.group_y), [rgrp] "s"(rgrp)
-                     : "v48", "v49", "v50", "v51", "v52", "v53", "v54", "v55", "v56", "v57", "vcc", "scc");
+                     : VRT_STEP_OUT(r.cur, r.side, g), [desc] "+&v"(r.descents), [gi] "+&v"(gi), [lanes] "=&s"(lanes)
+                     : VRT_STEP_IN(r.o, r.d, r.inv, r.ts, r.dm, bias, max_iters), [gz] "s"(w.group_z), [gy] "s"(w.group_y), [rgrp] "s"(rgrp)
+                     : VRT_STEP_CLOBBERS, "v56", "v57");
     } else {
         asm volatile("s_mov_b64 %[save], exec\n\t"
                      "s_branch vrt_look%=\n"
-                     "vrt_advance%=:\n\t" VRT_STEP_ADVANCE
+                     "vrt_advance%=:\n\t" VRT_STEP_ADVANCE("%[t0]", VRT_STEP_BIAS)
                      VRT_STEP_FLOOR "vrt_look%=:\n\t" VRT_STEP_SECTOR("%[alive]")
                      "s_cbranch_vccz vrt_advance%=\n\t" VRT_STEP_BRICK
                      "vrt_done%=:\n\t"
                      "s_mov_b64 exec, %[save]\n\t"
                      "v_mov_b32 %[base], v50"
-                     : VRT_STEP_OPERANDS
-                     : VRT_STEP_INPUTS
-                     : "v48", "v49", "v50", "v51", "v52", "v53", "v54", "v55", "vcc", "scc");
+                     : VRT_STEP_OUT(r.cur, r.side, g), [desc] "+&v"(r.descents)
+                     : VRT_STEP_IN(r.o, r.d, r.inv, r.ts, r.dm, bias, max_iters)
+                     : VRT_STEP_CLOBBERS);
     }
-#undef VRT_STEP_OPERANDS
-#undef VRT_STEP_INPUTS
     const bool hit = iters < max_iters && (int32_t)base >= 0;
     v[0] = (int32_t)(g[0] & 0x7FFFFFu) - kStepPad;
     v[1] = (int32_t)(g[1] & 0x7FFFFFu) - kStepPad;
@@ -611,7 +617,7 @@ template <bool GROUPS = false>
 __device__ __forceinline__ bool ray_trace_wave(const WorldView& w, RayState& r, uint32_t max_iters, int32_t v[3],
                                                uint32_t& slot, uint32_t first = 0) {
     const bool near = origin_is_guarded(r.W);  // uniform
-    if (!(near && __all(ray_is_quick(r)))) {
+    if (!(near && __all(ray_is_quick(r.o, r.d, r.inv)))) {
         ray_exact_inverse(r);
         if (!(near && __all(ray_is_tame(r) && ray_is_guarded(w, r))))
             return ray_trace_exact(w, r, max_iters, v, slot, first);

@@ -99,7 +99,8 @@ constexpr int32_t kStepPad = 128;
 //   w     per 2x2x2 group of bricks (gx, gz, gy = bit 4 of x, z, y) the cell mask of a step that
 //         stays at the sector level: bits 3..4 of w >> (2 gx + 8 gz + 16 gy) are bits 3..4 of that
 //         mask, whose bits 0..2 are always set: 7 when the group holds a brick, 15 when it is
-//         empty, 31 when the sector is
+//         empty, 31 when the sector is.  Bits 8..9 are the shader method's level above an empty
+//         sector (group_lod), 0 otherwise
 __host__ __device__ inline uint4 step_record(uint64_t mask, uint32_t base) {
     uint32_t codes = 0;
     for (uint32_t g = 0; g < 8; g++) {
@@ -109,6 +110,13 @@ __host__ __device__ inline uint4 step_record(uint64_t mask, uint32_t base) {
         codes |= code << (3 + 2 * gx + 8 * gz + 16 * gy);
     }
     return make_uint4((uint32_t)mask, (uint32_t)(mask >> 32), base, codes);
+}
+// The shader method steps 32, 64 or 128 voxels over an empty sector: 128 when the mask of its 4x4x4
+// sectors is 0, 64 when its 2x2x2 group of them is.  Code 0, 1 or 3 for sector x | z << 2 | y << 4:
+// bits 5..6 of the cell mask.
+__host__ __device__ inline uint32_t group_lod(uint64_t group, uint32_t sector) {
+    const uint32_t half = sector < 32 ? (uint32_t)group : (uint32_t)(group >> 32);
+    return group == 0 ? 3u : (((half >> (sector & 0xAu)) & 0x00330033u) == 0 ? 1u : 0u);
 }
 inline __host__ __device__ uint4 step_border_record() { return make_uint4(~0u, ~0u, ~0u, 0u); }
 

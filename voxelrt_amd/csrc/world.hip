@@ -186,7 +186,9 @@ __global__ __launch_bounds__(256) void step_tables_init_kernel(uint4* __restrict
         const uint32_t k = i < first ? 0u : i - first, ny = (step_n - first) / step_y;
         const uint32_t y = k / step_y, z = k % step_y / step_z, x = k % step_z;
         const bool border = x == 0 || x == step_z - 1 || z == 0 || z == step_z - 1 || y == 0 || y == ny - 1;
-        steps[i] = border ? step_border_record() : step_record(0, 0);
+        uint4 r = border ? step_border_record() : step_record(0, 0);
+        if (!border) r.w |= group_lod(0, 0) << 8;
+        steps[i] = r;
     }
     if (i < group_n) {
         const uint32_t y = i / group_y, z = i % group_y / group_z, x = i % group_z;
@@ -196,8 +198,7 @@ __global__ __launch_bounds__(256) void step_tables_init_kernel(uint4* __restrict
     }
 }
 
-// Records of the synced sectors (indices unique) and the sector-of-sectors words they changed, also
-// in the fast step's tables.
+// Records of the synced sectors (indices unique), in both tables.
 struct StepTables {
     uint4* steps;
     uint64_t* groups;
@@ -206,10 +207,7 @@ struct StepTables {
 };
 __global__ __launch_bounds__(256) void sync_records_kernel(uint4* __restrict__ sec, StepTables st,
                                                            const uint4* __restrict__ rec,
-                                                           const uint32_t* __restrict__ rec_idx, uint32_t nrec,
-                                                           uint64_t* __restrict__ groups,
-                                                           const uint64_t* __restrict__ gval,
-                                                           const uint32_t* __restrict__ gidx, uint32_t ngrp) {
+                                                           const uint32_t* __restrict__ rec_idx, uint32_t nrec) {
     uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i < nrec) {
         const uint32_t s = rec_idx[i], n1 = (1u << st.shift_xz) - 1u;
@@ -217,12 +215,28 @@ __global__ __launch_bounds__(256) void sync_records_kernel(uint4* __restrict__ s
         sec[s] = r;
         const uint32_t X = (s & n1) + 4u, Z = ((s >> st.shift_xz) & n1) + 4u, Y = (s >> (2 * st.shift_xz)) + 4u;
         st.steps[X + Z * st.step_z + Y * st.step_y] = step_record((uint64_t)r.x | (uint64_t)r.y << 32, r.z);
-    } else if (i - nrec < ngrp) {
-        const uint32_t g = gidx[i - nrec], n1 = (1u << st.gshift_xz) - 1u;
-        groups[g] = gval[i - nrec];
-        const uint32_t X = (g & n1) + 1u, Z = ((g >> st.gshift_xz) & n1) + 1u, Y = (g >> (2 * st.gshift_xz)) + 1u;
-        st.groups[X + Z * st.group_z + Y * st.group_y] = gval[i - nrec] | st.outside;
     }
+}
+
+// Changed sector-of-sectors words, thread (word, sector of it): the word goes to both tables, and
+// the empty sectors' step records get their level above the sector.  After the records.
+__global__ __launch_bounds__(256) void sync_groups_kernel(StepTables st, uint64_t* __restrict__ groups,
+                                                          const uint64_t* __restrict__ gval,
+                                                          const uint32_t* __restrict__ gidx, uint32_t ngrp) {
+    const uint32_t gid = blockIdx.x * blockDim.x + threadIdx.x, k = gid >> 6, b = gid & 63u;
+    if (k >= ngrp) return;
+    const uint32_t g = gidx[k], n1 = (1u << st.gshift_xz) - 1u;
+    const uint64_t m = gval[k];
+    const uint32_t gx = g & n1, gz = (g >> st.gshift_xz) & n1, gy = g >> (2 * st.gshift_xz);
+    if (b == 0) {
+        groups[g] = m;
+        st.groups[gx + 1u + (gz + 1u) * st.group_z + (gy + 1u) * st.group_y] = m | st.outside;
+    }
+    if (((m | st.outside) >> b) & 1u) return;
+    const uint32_t X = gx * 4u + (b & 3u) + 4u, Z = gz * 4u + ((b >> 2) & 3u) + 4u, Y = gy * 4u + (b >> 4) + 4u;
+    uint4 r = step_record(0, 0);
+    r.w |= group_lod(m, b) << 8;
+    st.steps[X + Z * st.step_z + Y * st.step_y] = r;
 }
 
 }  // namespace vrt
@@ -570,9 +584,12 @@ static int world_sync(vrt_world* w, uint32_t nsec, const uint32_t* sector_idx, c
         std::memcpy(hp + o_gidx, gidx.data() + g0, (size_t)ng * 4);
         e = hipMemcpyAsync(dp, hp, bytes, hipMemcpyHostToDevice, s);
         if (e == hipSuccess) {
-            sync_records_kernel<<<(nr + ng + 255) / 256, 256, 0, s>>>(
-                w->d_sec, st, (const uint4*)dp, (const uint32_t*)(dp + o_idx), nr, w->d_groups,
-                (const uint64_t*)(dp + o_gval), (const uint32_t*)(dp + o_gidx), ng);
+            if (nr)
+                sync_records_kernel<<<(nr + 255) / 256, 256, 0, s>>>(w->d_sec, st, (const uint4*)dp,
+                                                                     (const uint32_t*)(dp + o_idx), nr);
+            else
+                sync_groups_kernel<<<(uint32_t)(((uint64_t)ng * 64 + 255) / 256), 256, 0, s>>>(
+                    st, w->d_groups, (const uint64_t*)(dp + o_gval), (const uint32_t*)(dp + o_gidx), ng);
             e = hipGetLastError();
         }
         if (e == hipSuccess) e = release_half(w, h, s);
