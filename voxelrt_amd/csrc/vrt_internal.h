@@ -5,6 +5,7 @@
 
 #include <cstdint>
 #include <map>
+#include <mutex>
 #include <string>
 #include <vector>
 
@@ -80,7 +81,7 @@ private:
 // slot, and the cell mask of a step at the sector level whose 2x2x2 group of bricks
 // is empty: 15 (a 16-voxel cell), or 31 (the whole sector) when the mask is 0, the
 // reference's +2 LOD of an empty mask; a step whose group holds a brick uses half.
-inline uint4 sector_record(uint64_t mask, uint32_t base) {
+__host__ __device__ inline uint4 sector_record(uint64_t mask, uint32_t base) {
     return make_uint4((uint32_t)mask, (uint32_t)(mask >> 32), base, mask ? 15u : 31u);
 }
 
@@ -155,6 +156,7 @@ struct vrt_world {
     uint32_t log2_xz = 0, log2_y = 0;
     uint32_t shift_xz = 0, shift_y = 0;
     uint32_t nsec = 0;
+    uint8_t* d_tables = nullptr;      // one allocation for every table but d_occ and d_vox
     uint4* d_sec = nullptr;           // packed sector records (mask, base slot)
     uint4* d_steps = nullptr;         // the step table
     uint64_t* d_sgroups = nullptr;    // the group table
@@ -190,6 +192,10 @@ struct vrt_world {
     size_t moves_cap = 0;
     hipEvent_t moves_ev = nullptr;
     bool moves_pending = false;
+    // picking: the host memory its kernel writes its result to, and the last pick's number
+    void* h_pick = nullptr;
+    mutable std::mutex pick_mu;
+    mutable uint32_t pick_seq = 0;
     // totals since creation
     uint64_t upload_bytes = 0, upload_brick_bytes = 0, moved_bricks = 0;
 
@@ -240,6 +246,8 @@ struct vrt_world {
 };
 
 namespace vrt {
+// Bytes of a world's picking result.
+constexpr size_t kPickBytes = 64;
 // Bytes of one sync staging half (host pinned and device).
 constexpr size_t kSyncHalf = (size_t)8 << 20;
 

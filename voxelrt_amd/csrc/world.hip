@@ -176,26 +176,33 @@ __global__ __launch_bounds__(256) void sync_place_kernel(uint8_t* __restrict__ v
     for (int j = 0; j < 4; j++) d4[j] = s4[j];
 }
 
-// The step and group tables of an empty world: border records around records of empty sectors.
-__global__ __launch_bounds__(256) void step_tables_init_kernel(uint4* __restrict__ steps, uint32_t step_z,
-                                                               uint32_t step_y, uint32_t first, uint32_t step_n,
-                                                               uint64_t* __restrict__ groups, uint32_t group_z,
-                                                               uint32_t group_y, uint32_t group_n, uint64_t outside) {
-    uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < step_n) {
-        const uint32_t k = i < first ? 0u : i - first, ny = (step_n - first) / step_y;
-        const uint32_t y = k / step_y, z = k % step_y / step_z, x = k % step_z;
-        const bool border = x == 0 || x == step_z - 1 || z == 0 || z == step_z - 1 || y == 0 || y == ny - 1;
+// The tables of an empty world: records of empty sectors, in the step and group tables with a border
+// around them, no group bits and a zero palette.
+struct WorldTables {
+    uint4 *sec, *steps;
+    uint64_t *groups, *sgroups, *palette;
+    uint32_t nsec, step_z, step_y, step_first, step_n, ngroups, group_z, group_y, group_n;
+    uint64_t outside;
+};
+__global__ __launch_bounds__(256) void world_init_kernel(WorldTables t) {
+    const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
+    if (i < t.nsec) t.sec[i] = sector_record(0, 0);
+    if (i < t.step_n) {
+        const uint32_t k = i < t.step_first ? 0u : i - t.step_first, ny = (t.step_n - t.step_first) / t.step_y;
+        const uint32_t y = k / t.step_y, z = k % t.step_y / t.step_z, x = k % t.step_z;
+        const bool border = x == 0 || x == t.step_z - 1 || z == 0 || z == t.step_z - 1 || y == 0 || y == ny - 1;
         uint4 r = border ? step_border_record() : step_record(0, 0);
         if (!border) r.w |= group_lod(0, 0) << 8;
-        steps[i] = r;
+        t.steps[i] = r;
     }
-    if (i < group_n) {
-        const uint32_t y = i / group_y, z = i % group_y / group_z, x = i % group_z;
+    if (i < t.ngroups) t.groups[i] = 0;
+    if (i < t.group_n) {
+        const uint32_t y = i / t.group_y, z = i % t.group_y / t.group_z, x = i % t.group_z;
         const bool border =
-            x == 0 || x == group_z - 1 || z == 0 || z == group_z - 1 || y == 0 || y == group_n / group_y - 1;
-        groups[i] = border ? ~0ull : outside;
+            x == 0 || x == t.group_z - 1 || z == 0 || z == t.group_z - 1 || y == 0 || y == t.group_n / t.group_y - 1;
+        t.sgroups[i] = border ? ~0ull : t.outside;
     }
+    if (i < 256) t.palette[i] = 0;
 }
 
 // Records of the synced sectors (indices unique), in both tables.
@@ -277,17 +284,13 @@ static int grow_slots(vrt_world* w, uint32_t need, hipStream_t s) {
 }
 
 static void free_world(vrt_world* w) {
-    (void)hipFree(w->d_sec);
-    (void)hipFree(w->d_steps);
-    (void)hipFree(w->d_sgroups);
+    (void)hipFree(w->d_tables);
     (void)hipFree(w->d_occ);
     (void)hipFree(w->d_vox);
-    (void)hipFree(w->d_palette);
-    (void)hipFree(w->d_groups);
-    (void)hipFree(w->d_lut);
     (void)hipFree(w->d_stage);
     (void)hipFree(w->d_moves);
     if (w->h_stage) (void)hipHostFree(w->h_stage);
+    if (w->h_pick) (void)hipHostFree(w->h_pick);
     for (hipEvent_t e : w->stage_ev)
         if (e) (void)hipEventDestroy(e);
     if (w->moves_ev) (void)hipEventDestroy(w->moves_ev);
@@ -662,23 +665,33 @@ int vrt_world_create(const vrt_world_desc* desc, void* stream, vrt_world** out) 
         auto check = [&](hipError_t e, const char* what) {
             if (e != hipSuccess && rc == VRT_OK) rc = hip_fail(e, what);
         };
-        check(hipMalloc(&w->d_sec, (size_t)w->nsec * 16), "hipMalloc(sector records)");
-        check(hipMalloc(&w->d_steps, (size_t)w->step_n() * 16), "hipMalloc(step table)");
-        check(hipMalloc(&w->d_sgroups, (size_t)w->group_n() * 8), "hipMalloc(group table)");
-        check(hipMalloc(&w->d_palette, 256 * 8), "hipMalloc(palette)");
-        check(hipMalloc(&w->d_groups, w->h_groups.size() * 8), "hipMalloc(sector groups)");
-        check(hipMalloc(&w->d_lut, 512 * 8), "hipMalloc(ray-cell table)");
+        // one allocation for the tables, each at a multiple of 256 bytes
+        size_t bytes = 0;
+        auto part = [&](size_t n) {
+            const size_t at = bytes;
+            bytes += (n + 255) & ~(size_t)255;
+            return at;
+        };
+        const size_t o_sec = part((size_t)w->nsec * 16), o_steps = part((size_t)w->step_n() * 16);
+        const size_t o_groups = part(w->h_groups.size() * 8), o_sgroups = part((size_t)w->group_n() * 8);
+        const size_t o_palette = part(256 * 8), o_lut = part(512 * 8);
+        check(hipMalloc(&w->d_tables, bytes), "hipMalloc(world tables)");
+        check(hipHostMalloc(&w->h_pick, kPickBytes, hipHostMallocDefault), "hipHostMalloc(picking result)");
         if (rc == VRT_OK) {
-            std::vector<uint4> empty(w->nsec, sector_record(0, 0));
-            check(hipMemcpyAsync(w->d_sec, empty.data(), (size_t)w->nsec * 16, hipMemcpyHostToDevice, s),
-                  "hipMemcpyAsync(sector records)");
-            step_tables_init_kernel<<<(std::max(w->step_n(), w->group_n()) + 255) / 256, 256, 0, s>>>(
-                w->d_steps, w->step_z(), w->step_y(), w->step_first(), w->step_n(), w->d_sgroups, w->group_z(),
-                w->group_y(), w->group_n(), w->group_outside());
-            check(hipGetLastError(), "step_tables_init_kernel");
-            check(hipStreamSynchronize(s), "hipStreamSynchronize(sector records)");
-            check(hipMemsetAsync(w->d_palette, 0, 256 * 8, s), "hipMemsetAsync(palette)");
-            check(hipMemsetAsync(w->d_groups, 0, w->h_groups.size() * 8, s), "hipMemsetAsync(sector groups)");
+            std::memset(w->h_pick, 0, kPickBytes);
+            w->d_sec = (uint4*)(w->d_tables + o_sec);
+            w->d_steps = (uint4*)(w->d_tables + o_steps);
+            w->d_groups = (uint64_t*)(w->d_tables + o_groups);
+            w->d_sgroups = (uint64_t*)(w->d_tables + o_sgroups);
+            w->d_palette = (uint64_t*)(w->d_tables + o_palette);
+            w->d_lut = (uint64_t*)(w->d_tables + o_lut);
+            const WorldTables t{w->d_sec,       w->d_steps,     w->d_groups, w->d_sgroups, w->d_palette,
+                                w->nsec,        w->step_z(),    w->step_y(), w->step_first(), w->step_n(),
+                                (uint32_t)w->h_groups.size(),   w->group_z(), w->group_y(), w->group_n(),
+                                w->group_outside()};
+            const uint32_t n = std::max({w->nsec, w->step_n(), w->group_n(), 256u});
+            world_init_kernel<<<(n + 255) / 256, 256, 0, s>>>(t);
+            check(hipGetLastError(), "world_init_kernel");
             check(hipMemcpyAsync(w->d_lut, lut.data(), 512 * 8, hipMemcpyHostToDevice, s), "hipMemcpyAsync(ray-cell table)");
         }
         if (rc == VRT_OK && desc->initial_slots) rc = grow_slots(w, std::min(desc->initial_slots, w->arena.capacity()), s);
