@@ -140,20 +140,39 @@ __global__ __launch_bounds__(256) void render_bwd_kernel(uint32_t n, const float
 
 // ---------------------------------------------------------------- brick-bucketed backward
 
-// The whole gradient written once, with no global float atomics: hit pixels are bucketed by
-// brick slot (a counting sort: per-slot counts with wave-aggregated integer atomics, a
-// two-level exclusive scan, a placement pass), then one wave per slot sums its pixels'
-// contributions in LDS and writes the slot's 512 x 3 gradient entries, zeros for a slot no
-// pixel hit.  On the 16 views of the 512^3 terrain, 2.2 M hit pixels land on 287 k voxels,
-// 7.8 pixels per voxel across views, so per-pixel global atomics contend, and a dense
-// gradient zeroed first is written twice.
-constexpr uint32_t kScanBlock = 1024;  // counts per block of the two-level scan
+// Hit pixels are bucketed by brick slot (a counting sort: per-slot counts with wave-aggregated integer
+// atomics, an allocation of the slots' lists, a placement pass), then a workgroup per touched slot
+// sums its pixels' contributions in LDS and writes the slot's 512 x 3 gradient entries: no global
+// float atomics.  The other entries are zeros, and they are most of it: 16 views of 512 x 512 over the
+// 512^3 terrain touch 8.9 k of its 97 k slots (1.7 M pixels, 195 per touched slot).  So the gradient is
+// filled with zeros first, at the rate of a fill, and the touched slots are written a second time.
+// Measured there (598 MB), in us: fill 77, counts 33, allocation 5, placement 24, sums 19, against 197
+// for six launches the last of which wrote each slot's zeros or sums by a wave.  Sharing a launch
+// between the fill and the counts or the placement gained nothing (they wait for each other's memory),
+// nor did filling after the placement (counts and placement 8 faster, sums 5 slower, a launch more).
+constexpr uint32_t kScanBlock = 1024;   // slots per block of the allocation
+
+// Zeros in `vecs` float4s from `out` and the `tail` floats after them, and in `n` words of p.  A float4
+// per thread, so that neighbouring blocks fill neighbouring 4 KB: 6.9 TB/s (blocks of 16 and 64 KB
+// reach 6.1 and 5.1, grids that stride over the gradient 4.4-6.1).
+__global__ __launch_bounds__(256) void bwd_fill_kernel(float4* __restrict__ out, uint64_t vecs, uint32_t tail,
+                                                       uint32_t* __restrict__ p, uint32_t n) {
+    const uint64_t v = (uint64_t)blockIdx.x * 256 + threadIdx.x;
+    if (v < vecs)
+        out[v] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+    else if (v - vecs < tail)
+        ((float*)(out + vecs))[v - vecs] = 0.0f;
+    else if (v - vecs - tail < n)
+        p[v - vecs - tail] = 0u;
+}
 
 // Pass 1: the rank of each contributing pixel among the pixels of its slot; counts[slot] ends
 // as the slot's pixel count.  Lanes of a wave with the same slot share one atomic (each round
 // matches the first pending lane's slot by ballot; a lane's rank is its position among the
 // matches).  Eight rounds, unrolled with one result variable each, so a wave's atomics are all
-// in flight together and the wave waits for their returns once, after the last round.
+// in flight together and the wave waits for their returns once, after the last round.  Bound by the
+// atomics, which are performed past the XCDs' L2s, 23 to an address here: with four rows of pixels in
+// flight per wave it took 42 us and not 30.
 __global__ __launch_bounds__(256) void bwd_count_kernel(uint32_t n, const uint32_t* __restrict__ saved_voxel,
                                                         const float* __restrict__ saved_weight,
                                                         uint32_t* __restrict__ counts, uint32_t* __restrict__ rank) {
@@ -205,140 +224,123 @@ __global__ __launch_bounds__(256) void bwd_count_kernel(uint32_t n, const uint32
     if (i < n) rank[i] = r;
 }
 
-// Pass 2a: exclusive scan of counts inside blocks of kScanBlock (256 threads x 4), into offsets;
-// block_sum[b] = the block's total.
-__global__ __launch_bounds__(256) void bwd_scan_blocks_kernel(uint32_t nb, const uint32_t* __restrict__ counts,
-                                                              uint32_t* __restrict__ offsets,
-                                                              uint32_t* __restrict__ block_sum) {
-    __shared__ uint32_t wave_total[4];
+// Pass 2: the slots' lists and the list of the touched slots.  A block scans kScanBlock counts
+// (256 threads x 4) and takes its room in both lists with one atomic each, so the lists' order
+// varies between runs, as the ranks do.
+__global__ __launch_bounds__(256) void bwd_alloc_kernel(uint32_t ns, const uint32_t* __restrict__ counts,
+                                                        uint32_t* __restrict__ cursor, uint32_t* __restrict__ offsets,
+                                                        uint4* __restrict__ touched) {
+    __shared__ uint64_t wave_total[4];
+    __shared__ uint32_t start[2];
     const uint32_t t = threadIdx.x, lane = t & 63u, wave = t >> 6;
     const uint32_t base = blockIdx.x * kScanBlock + t * 4;
-    uint32_t c[4], sum = 0;
+    uint32_t c[4];
+    uint64_t sum = 0;  // pixels, and touched slots in the high half (a block holds at most 2^10)
 #pragma unroll
     for (int k = 0; k < 4; k++) {
-        c[k] = base + k < nb ? counts[base + k] : 0u;
-        sum += c[k];
+        c[k] = base + k < ns ? counts[base + k] : 0u;
+        sum += (uint64_t)c[k] | (uint64_t)(c[k] != 0) << 32;
     }
-    uint32_t incl = sum;
+    uint64_t incl = sum;
 #pragma unroll
     for (uint32_t off = 1; off < 64; off <<= 1) {
-        uint32_t y = __shfl_up(incl, off, 64);
+        uint64_t y = __shfl_up((unsigned long long)incl, off, 64);
         if (lane >= off) incl += y;
     }
     if (lane == 63) wave_total[wave] = incl;
     __syncthreads();
-    uint32_t run = incl - sum;
+    uint64_t run = incl - sum;
     for (uint32_t w = 0; w < wave; w++) run += wave_total[w];
+    if (t == 255) {
+        const uint64_t total = run + sum;
+        start[0] = (uint32_t)total ? atomicAdd(&cursor[0], (uint32_t)total) : 0u;
+        start[1] = (uint32_t)total ? atomicAdd(&cursor[1], (uint32_t)(total >> 32)) : 0u;
+    }
+    __syncthreads();
+    uint32_t px = start[0] + (uint32_t)run, ts = start[1] + (uint32_t)(run >> 32);
 #pragma unroll
     for (int k = 0; k < 4; k++) {
-        if (base + k < nb) offsets[base + k] = run;
-        run += c[k];
-    }
-    if (t == 255) block_sum[blockIdx.x] = run;
-}
-
-// Pass 2b: exclusive scan of the block totals in one workgroup (runs of consecutive totals per
-// thread, combined across the 16 waves).
-__global__ __launch_bounds__(1024) void bwd_scan_totals_kernel(uint32_t nblk, uint32_t* __restrict__ block_sum) {
-    __shared__ uint32_t wave_total[16];
-    const uint32_t t = threadIdx.x, lane = t & 63u, wave = t >> 6;
-    uint32_t per = (nblk + 1023) / 1024;
-    uint32_t begin = min(t * per, nblk), end = min(begin + per, nblk);
-    uint32_t sum = 0;
-    for (uint32_t k = begin; k < end; k++) sum += block_sum[k];
-    uint32_t incl = sum;
-#pragma unroll
-    for (uint32_t off = 1; off < 64; off <<= 1) {
-        uint32_t y = __shfl_up(incl, off, 64);
-        if (lane >= off) incl += y;
-    }
-    if (lane == 63) wave_total[wave] = incl;
-    __syncthreads();
-    uint32_t run = incl - sum;
-    for (uint32_t w = 0; w < wave; w++) run += wave_total[w];
-    for (uint32_t k = begin; k < end; k++) {
-        uint32_t c = block_sum[k];
-        block_sum[k] = run;
-        run += c;
+        if (c[k] == 0) continue;
+        offsets[base + k] = px;
+        touched[ts++] = make_uint4(base + k, px, c[k], 0u);
+        px += c[k];
     }
 }
 
-// Pass 3: each contributing pixel's index at its slot's offset plus its rank.
-__global__ __launch_bounds__(256) void bwd_place_kernel(uint32_t n, const uint32_t* __restrict__ saved_voxel,
-                                                        const uint32_t* __restrict__ rank,
-                                                        const uint32_t* __restrict__ offsets,
-                                                        const uint32_t* __restrict__ block_sum,
-                                                        uint32_t* __restrict__ list) {
-    uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= n) return;
-    uint32_t r = rank[i];
-    if (r == 0xFFFFFFFFu) return;
-    uint32_t slot = saved_voxel[i] >> 9;
-    list[offsets[slot] + block_sum[slot / kScanBlock] + r] = i;
-}
-
-// Pass 4: one wave per slot.  The slot's pixels add grad_image * weight into 512 x 3 LDS
-// accumulators (LDS float atomics), then the wave writes the slot's rows [slot * 512,
-// min(nvox, slot * 512 + 512)) of the gradient: every entry is written, zeros where no pixel hit.
-// On the 512^3 terrain's 97 k slots this moves 598 MB of gradient and ~145 MB of gathered pixel
-// data in 0.133 ms (5.6 TB/s); four slots per workgroup (0.145 ms) and a grid stride over 8192
-// long-lived waves (0.156 ms) measured slower.  The gradient rows are written with non-temporal
-// stores (nothing in the pass reads them back): 2% off the backward in alternating runs.
-__device__ __forceinline__ void store_row4_nt(float4* dst, float4 x) {
-    float* q = (float*)dst;
-    __builtin_nontemporal_store(x.x, q + 0);
-    __builtin_nontemporal_store(x.y, q + 1);
-    __builtin_nontemporal_store(x.z, q + 2);
-    __builtin_nontemporal_store(x.w, q + 3);
-}
-
-__global__ __launch_bounds__(64) void bwd_reduce_kernel(uint64_t nvox, const float* __restrict__ grad_image,
+// Pass 3: each contributing pixel's contribution, grad_image * weight, and voxel as one 16-byte entry at
+// its slot's offset plus its rank.  (With the pixel's index there instead, 11 us and not 24, the next
+// pass gathers the pixels' data and takes 39 us and not 19: a slot's pixels are runs of 8 or so in an
+// 8x8 tile, and most of each line fetched for them belongs to other slots.)
+__global__ __launch_bounds__(256) void bwd_place_kernel(uint32_t n, const float* __restrict__ grad_image,
                                                         const uint32_t* __restrict__ saved_voxel,
                                                         const float* __restrict__ saved_weight,
-                                                        const uint32_t* __restrict__ counts,
+                                                        const uint32_t* __restrict__ rank,
                                                         const uint32_t* __restrict__ offsets,
-                                                        const uint32_t* __restrict__ block_sum,
-                                                        const uint32_t* __restrict__ list,
-                                                        float* __restrict__ grad_albedo) {
-    __shared__ float acc[512 * 3];
-    const uint32_t slot = blockIdx.x, lane = threadIdx.x;
-    const uint64_t row0 = (uint64_t)slot * 512;
-    const uint32_t rows = (uint32_t)min<uint64_t>(512, nvox - row0);
-    float* out = grad_albedo + row0 * 3;
-    const uint32_t cnt = counts[slot];
-    if (cnt == 0) {
-        if (rows == 512) {
-            float4* o4 = (float4*)out;
-            for (uint32_t k = lane; k < 384; k += 64) store_row4_nt(&o4[k], make_float4(0.0f, 0.0f, 0.0f, 0.0f));
-        } else {
-            for (uint32_t k = lane; k < rows * 3; k += 64) out[k] = 0.0f;
-        }
-        return;
-    }
-    for (uint32_t k = lane; k < 512 * 3; k += 64) acc[k] = 0.0f;
-    __syncthreads();
-    const uint32_t begin = offsets[slot] + block_sum[slot / kScanBlock];
-    for (uint32_t j = lane; j < cnt; j += 64) {
-        uint32_t p = list[begin + j];
-        uint32_t v = saved_voxel[p] & 511u;
-        float w = saved_weight[p];
-        atomicAdd(&acc[v * 3 + 0], grad_image[(size_t)p * 3 + 0] * w);
-        atomicAdd(&acc[v * 3 + 1], grad_image[(size_t)p * 3 + 1] * w);
-        atomicAdd(&acc[v * 3 + 2], grad_image[(size_t)p * 3 + 2] * w);
-    }
-    __syncthreads();
-    if (rows == 512) {
-        float4* o4 = (float4*)out;
-        const float4* a4 = (const float4*)acc;
-        for (uint32_t k = lane; k < 384; k += 64) store_row4_nt(&o4[k], a4[k]);
-    } else {
-        for (uint32_t k = lane; k < rows * 3; k += 64) out[k] = acc[k];
-    }
+                                                        float4* __restrict__ list) {
+    const uint32_t i = blockIdx.x * 256 + threadIdx.x;
+    if (i >= n) return;
+    const uint32_t r = rank[i], gv = saved_voxel[i];
+    const float w = saved_weight[i];
+    const float x = grad_image[(size_t)i * 3 + 0] * w, y = grad_image[(size_t)i * 3 + 1] * w,
+                z = grad_image[(size_t)i * 3 + 2] * w;
+    if (r != 0xFFFFFFFFu) list[offsets[gv >> 9] + r] = make_float4(x, y, z, __uint_as_float(gv & 511u));
 }
 
-__global__ void bwd_fill_kernel(uint32_t* p, uint32_t n) {
-    uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < n) p[i] = 0u;
+// Pass 4: one workgroup per touched slot, striding over them (their number is on the device).  The
+// slot's entries are added into 512 x 3 LDS accumulators, then the workgroup writes the slot's rows
+// [slot * 512, min(nvox, slot * 512 + 512)) of the gradient.  The accumulators are doubles: an LDS
+// atomic add of 64 floats takes this part 194 cycles, of doubles 18-22 (the adds alone held this pass
+// at 50 us with floats), and the sums are rounded once.  Bound by latency: the next slot's place is
+// loaded ahead, and a thread has kReducePixels entries in flight.  Each XCD (workgroup b runs on XCD
+// b % 8) takes an eighth of the slots in a piece.
+constexpr uint32_t kReduceThreads = 128;
+constexpr uint32_t kReduceBlocks = 3072;  // 12 per CU: 12 KB of LDS each, of 160
+constexpr uint32_t kReducePixels = 2;
+
+__global__ __launch_bounds__(kReduceThreads) void bwd_reduce_kernel(uint64_t nvox,
+                                                                    const uint32_t* __restrict__ cursor,
+                                                                    const uint4* __restrict__ touched,
+                                                                    const float4* __restrict__ list,
+                                                                    float* __restrict__ grad_albedo) {
+    __shared__ __align__(16) double acc[512 * 3];
+    const uint32_t t = threadIdx.x, ntouched = cursor[1];
+    const uint32_t per = (ntouched + 7) / 8, first = (blockIdx.x & 7u) * per, end = min(first + per, ntouched);
+    uint32_t s = first + (blockIdx.x >> 3);
+    if (s >= end) return;
+    uint4 next = touched[s];
+    while (s < end) {
+        const uint32_t slot = next.x, begin = next.y, cnt = next.z;
+        s += gridDim.x >> 3;
+        if (s < end) next = touched[s];  // ahead of its use
+        for (uint32_t k = t; k < 768; k += kReduceThreads) ((double2*)acc)[k] = make_double2(0.0, 0.0);
+        __syncthreads();
+        for (uint32_t j0 = 0; j0 < cnt; j0 += kReduceThreads * kReducePixels) {
+            float4 e[kReducePixels];
+#pragma unroll
+            for (uint32_t q = 0; q < kReducePixels; q++)
+                e[q] = list[begin + min(j0 + q * kReduceThreads + t, cnt - 1u)];
+#pragma unroll
+            for (uint32_t q = 0; q < kReducePixels; q++) {
+                if (j0 + q * kReduceThreads + t >= cnt) continue;
+                double* a = acc + __float_as_uint(e[q].w) * 3;
+                atomicAdd(a + 0, (double)e[q].x);
+                atomicAdd(a + 1, (double)e[q].y);
+                atomicAdd(a + 2, (double)e[q].z);
+            }
+        }
+        __syncthreads();
+        const uint64_t row0 = (uint64_t)slot * 512;
+        const uint32_t rows = (uint32_t)min<uint64_t>(512, nvox - row0);
+        float* out = grad_albedo + row0 * 3;
+        if (rows == 512) {
+            for (uint32_t k = t; k < 384; k += kReduceThreads)
+                ((float4*)out)[k] = make_float4((float)acc[k * 4], (float)acc[k * 4 + 1], (float)acc[k * 4 + 2],
+                                                (float)acc[k * 4 + 3]);
+        } else {
+            for (uint32_t k = t; k < rows * 3; k += kReduceThreads) out[k] = (float)acc[k];
+        }
+        __syncthreads();
+    }
 }
 
 // Sparse gradient: entry p is (voxel id, grad_image[p] * weight[p]), or (0, 0) for a pixel that
@@ -358,29 +360,32 @@ __global__ __launch_bounds__(256) void bwd_sparse_kernel(uint32_t n, const float
     values[(size_t)i * 3 + 2] = take ? grad_image[(size_t)i * 3 + 2] * w : 0.0f;
 }
 
-// Workspace of the brick-bucketed backward: counts, offsets (one u32 per slot each), block
-// totals (one per kScanBlock slots), ranks and the pixel list (one u32 per pixel each), each
-// part 256-byte aligned.
+// Workspace of the brick-bucketed backward: two cursors and the counts (cleared together), offsets
+// (one u32 per slot each), the touched slots (slot, first entry, count), ranks (one u32 per pixel)
+// and the entries (16 bytes per pixel), each part 256-byte aligned.
 struct BwdWorkspace {
-    uint32_t *counts, *offsets, *block_sum, *rank, *list;
+    uint32_t *cursor, *counts, *offsets, *rank;
+    uint4* touched;
+    float4* list;
 };
+constexpr uint32_t kCursorWords = 64;  // before the counts
 
 static size_t align256(size_t x) { return (x + 255) & ~(size_t)255; }
 
 static size_t bwd_workspace_bytes(uint32_t npixels, uint64_t nslots) {
-    uint64_t nblk = (nslots + kScanBlock - 1) / kScanBlock;
-    return 2 * align256(nslots * 4) + align256(nblk * 4) + 2 * align256((size_t)npixels * 4);
+    return kCursorWords * 4 + 2 * align256(nslots * 4) + std::min<uint64_t>(nslots, npixels) * 16 + 256 +
+           align256((size_t)npixels * 4) + align256((size_t)npixels * 16);
 }
 
 static BwdWorkspace carve_bwd(void* base, uint32_t npixels, uint64_t nslots) {
-    uint64_t nblk = (nslots + kScanBlock - 1) / kScanBlock;
     char* p = (char*)base;
     BwdWorkspace ws;
+    ws.cursor = (uint32_t*)p; p += kCursorWords * 4;
     ws.counts = (uint32_t*)p; p += align256(nslots * 4);
     ws.offsets = (uint32_t*)p; p += align256(nslots * 4);
-    ws.block_sum = (uint32_t*)p; p += align256(nblk * 4);
+    ws.touched = (uint4*)p; p += align256(std::min<uint64_t>(nslots, npixels) * 16);
     ws.rank = (uint32_t*)p; p += align256((size_t)npixels * 4);
-    ws.list = (uint32_t*)p;
+    ws.list = (float4*)p;
     return ws;
 }
 
@@ -485,15 +490,20 @@ int vrt_render_bwd_bricks(const vrt_world* world, uint32_t npixels, const float*
         hipStream_t s = (hipStream_t)stream;
         BwdWorkspace ws = carve_bwd(workspace, npixels, nslots);
         const uint32_t ns = (uint32_t)nslots, nblk = (uint32_t)((nslots + kScanBlock - 1) / kScanBlock);
-        bwd_fill_kernel<<<(ns + 255) / 256, 256, 0, s>>>(ws.counts, ns);  // a kernel, not a memset (graph-safe)
-        if (npixels) bwd_count_kernel<<<(npixels + 255) / 256, 256, 0, s>>>(npixels, saved_voxel, saved_weight,
-                                                                            ws.counts, ws.rank);
-        bwd_scan_blocks_kernel<<<nblk, 256, 0, s>>>(ns, ws.counts, ws.offsets, ws.block_sum);
-        bwd_scan_totals_kernel<<<1, 1024, 0, s>>>(nblk, ws.block_sum);
-        if (npixels) bwd_place_kernel<<<(npixels + 255) / 256, 256, 0, s>>>(npixels, saved_voxel, ws.rank, ws.offsets,
-                                                                            ws.block_sum, ws.list);
-        bwd_reduce_kernel<<<ns, 64, 0, s>>>(nvox, grad_image, saved_voxel, saved_weight, ws.counts, ws.offsets,
-                                            ws.block_sum, ws.list, grad_albedo);
+        // kernels, not memsets (graph-safe); the counts and cursors are cleared with the gradient
+        const uint64_t vecs = nvox * 3 / 4;
+        const uint32_t tail = (uint32_t)(nvox * 3 % 4), words = npixels ? ns + kCursorWords : 0u;
+        bwd_fill_kernel<<<(uint32_t)((vecs + tail + words + 255) / 256), 256, 0, s>>>((float4*)grad_albedo, vecs, tail,
+                                                                                     ws.cursor, words);
+        if (npixels) {
+            bwd_count_kernel<<<(npixels + 255) / 256, 256, 0, s>>>(npixels, saved_voxel, saved_weight, ws.counts, ws.rank);
+            bwd_alloc_kernel<<<nblk, 256, 0, s>>>(ns, ws.counts, ws.cursor, ws.offsets, ws.touched);
+            bwd_place_kernel<<<(npixels + 255) / 256, 256, 0, s>>>(npixels, grad_image, saved_voxel, saved_weight, ws.rank,
+                                                                   ws.offsets, ws.list);
+            const uint32_t blocks = std::min({ns, npixels, kReduceBlocks});
+            bwd_reduce_kernel<<<(blocks + 7) / 8 * 8, kReduceThreads, 0, s>>>(nvox, ws.cursor, ws.touched, ws.list,
+                                                                             grad_albedo);
+        }
         VRT_HIP(hipGetLastError());
         return VRT_OK;
     });
