@@ -53,6 +53,8 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(7))) void re
     uint32_t tx = reverse ? gridDim.x - 1u - blockIdx.x : blockIdx.x;
     uint32_t ty = reverse ? gridDim.y - 1u - blockIdx.y : blockIdx.y;
     uint32_t px = tx * 8 + (threadIdx.x & 7u), py = ty * 8 + (threadIdx.x >> 3);
+    __shared__ uint4 lds_lut[LUT ? kLutPairs : 1];
+    const uint32_t lut = fill_lut<LUT>(sv, lds_lut);
     if (px >= a.cam.width || py >= a.cam.height) return;
     const uint32_t i = py * a.cam.width + px;
     const int32_t* W = a.cam.world_origin;
@@ -63,7 +65,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(7))) void re
     float albedo[3] = {1.0f, 1.0f, 1.0f}, irr[3], N[3] = {0.0f, 0.0f, 0.0f}, dep = -1.0f;
     ShaderHit hit;
     uint32_t iters;
-    if (shader_trace<false, LUT>(sv, a.cam.eye, rd, W, 256u, hit)) {
+    if (shader_trace<false, LUT>(sv, lut, a.cam.eye, rd, W, 256u, hit)) {
         iters = hit.iters;
         uint64_t mat = a.palette[hit.mat];
         material_color(mat, albedo);
@@ -95,7 +97,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(7))) void re
                 ro[c] = pos[c] + N[c] * 0.01f;
                 dir[c] = sun ? a.sun[c] : nudge_zero(dir[c]);
             }
-            const bool h = shader_trace<true, LUT>(sv, ro, dir, W, 96u, hit);
+            const bool h = shader_trace<true, LUT>(sv, lut, ro, dir, W, 96u, hit);
             if (sun) {
                 if (k == 0) {
 #pragma unroll

@@ -13,12 +13,14 @@ namespace {
 template <bool COARSE, bool LUT>
 __global__ __launch_bounds__(256) void shader_cast_kernel(ShaderView sv, RaysIn r, HitsOut h, uint32_t cap) {
     uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
+    __shared__ uint4 lds_lut[LUT ? kLutPairs : 1];
+    const uint32_t lut = fill_lut<LUT>(sv, lds_lut);
     if (i >= r.n) return;
     const float o[3] = {r.ox[i], r.oy[i], r.oz[i]};
     const float d[3] = {r.dx[i], r.dy[i], r.dz[i]};
     const int32_t W[3] = {r.W[0], r.W[1], r.W[2]};
     ShaderHit sh;
-    bool hit = shader_trace<COARSE, LUT>(sv, o, d, W, cap, sh);
+    bool hit = shader_trace<COARSE, LUT>(sv, lut, o, d, W, cap, sh);
     h.t[i] = sh.t;
     h.rec[i] = make_int4(sh.v[0], sh.v[1], sh.v[2], (int)(sh.mat | sh.code << 8 | (sh.iters & 0xFFFFu) << 16));
     if (h.pos_x) {

@@ -31,9 +31,9 @@ __device__ __forceinline__ void first_occupied(uint64_t m, int32_t v[3]) {
 // getStepPos (:92-131).  Returns true when v is solid (or, for a coarse step, when v
 // was moved to the first solid voxel of its non-empty 4x4x4 cell); otherwise moves v
 // to the far corner, in ray direction, of the largest empty aligned cell.
-template <bool LUT, bool TAME>
-__device__ __forceinline__ bool shader_step(const ShaderView& sv, int32_t v[3], const float d[3],
-                                            const int32_t dm[3], uint32_t oct, bool coarse) {
+template <bool LUT>
+__device__ __forceinline__ bool shader_step(const ShaderView& sv, int32_t v[3], const float d[3], uint32_t oct,
+                                            bool coarse) {
     const WorldView& w = sv.w;
     uint32_t ux = (uint32_t)v[0], uy = (uint32_t)v[1], uz = (uint32_t)v[2];
     uint32_t sx = ux >> 5, sy = uy >> 5, sz = uz >> 5;
@@ -71,13 +71,10 @@ __device__ __forceinline__ bool shader_step(const ShaderView& sv, int32_t v[3], 
         first_occupied(m, v);
         return true;
     }
-    // d < 0: v & ~cm, else v | cm (the fast loop: one bitfield insert of dm, all ones unless
-    // d < 0)
     uint32_t cm = (uint32_t)lod - 1u;
 #pragma unroll
     for (int a = 0; a < 3; a++)
-        v[a] = TAME ? (int32_t)bitfield_insert(~cm, (uint32_t)v[a], (uint32_t)dm[a])
-                    : (d[a] < 0.0f ? (int32_t)((uint32_t)v[a] & ~cm) : (int32_t)((uint32_t)v[a] | cm));
+        v[a] = d[a] < 0.0f ? (int32_t)((uint32_t)v[a] & ~cm) : (int32_t)((uint32_t)v[a] | cm);
     return false;
 }
 
@@ -111,15 +108,12 @@ struct ShaderHit {
     uint32_t mat;   // material id, 0 on a miss
 };
 
-// The loop of rayCast / rayCastCoarse.  TAME (every active ray of the wave has finite
-// 1/d and tStart, |origin| < 2^20 and 0.25 <= |d|^2 <= 4): positions stay far inside int32
-// range for any cap (a step moves less than 128 sqrt(3) / 0.5 voxels) and tmin is never NaN,
-// so floor is one V_CVT_FLR_I32_F32 instead of floor2i's range test.
-template <bool COARSE, bool LUT, bool TAME>
+// The loop of rayCast / rayCastCoarse for any ray.
+template <bool COARSE, bool LUT>
 __device__ __forceinline__ bool shader_loop(const ShaderView& sv, const float d[3], const float org[3],
-                                            const float inv[3], const float ts[3], const int32_t W[3],
-                                            const int32_t dm[3], uint32_t oct, uint32_t cap, int32_t v[3],
-                                            float side[3], float cur[3], float& tmin, uint32_t& it) {
+                                            const float inv[3], const float ts[3], const int32_t W[3], uint32_t oct,
+                                            uint32_t cap, int32_t v[3], float side[3], float cur[3], float& tmin,
+                                            uint32_t& it) {
     const WorldView& w = sv.w;
     bool hit = false;
     for (; it < cap; it++) {
@@ -134,10 +128,10 @@ __device__ __forceinline__ bool shader_loop(const ShaderView& sv, const float d[
 #pragma unroll
         for (int a = 0; a < 3; a++) {
             cur[a] = fmaf(tmin, d[a], org[a]);
-            v[a] = (int32_t)((uint32_t)W[a] + (uint32_t)(TAME ? floor_i32_in_range(cur[a]) : floor2i(cur[a])));
+            v[a] = (int32_t)((uint32_t)W[a] + (uint32_t)floor2i(cur[a]));
         }
         if (!((uint32_t)(v[0] | v[2]) < w.size_xz && (uint32_t)v[1] < w.size_y)) break;
-        if (shader_step<LUT, TAME>(sv, v, d, dm, oct, COARSE && it > 30)) {
+        if (shader_step<LUT>(sv, v, d, oct, COARSE && it > 30)) {
             hit = true;
             break;
         }
@@ -145,19 +139,91 @@ __device__ __forceinline__ bool shader_loop(const ShaderView& sv, const float d[
     return hit;
 }
 
-// shader_loop without the ray-cell table for quick rays (ray_is_quick of the start org, d and inv), in
-// worlds of at least 128 voxels on every axis: the cast's fast loop (traverse.h) with this method's
-// bias, its level above an empty sector (step records' bits 8..9) and rayCastCoarse's stop in a
-// non-empty cell from step 31 on.  The largest cell, 128 voxels, then lies inside the world, so
-// positions stay within the tables' border as there.  A step at the sector level takes 36 vector
+// The ray-cell table in a block's LDS, entry oct * 64 + (63 - cell): filled by all of its lanes, each
+// a pair of entries at a time, before the first trace.
+constexpr uint32_t kLutPairs = 256;
+template <bool LUT>
+__device__ __forceinline__ uint32_t fill_lut(const ShaderView& sv, uint4* lut) {
+    if constexpr (LUT) {
+        for (uint32_t p = threadIdx.x; p < kLutPairs; p += blockDim.x) {
+            const uint4 e = ((const uint4*)sv.lut)[p];
+            lut[p ^ 31u] = make_uint4(e.z, e.w, e.x, e.y);
+        }
+        __syncthreads();
+        return (uint32_t)(uintptr_t)(__attribute__((address_space(3))) uint4*)lut;
+    }
+    return 0;
+}
+
+// The masked mask v[54:55] of the cell with shifts t1 (its bit, from the top) and t2 (its 2x2x2
+// group): the ray-cell table's word, read before the mask arrives (VRT_LUT_READ), and as t0 and t1 the
+// mask ored and its 2x2x2 group's (VRT_LUT_MASK).
+#define VRT_LUT_READ                                       \
+    "v_and_b32 %[t0], 63, %[t1]\n\t"                       \
+    "v_lshl_add_u32 %[t0], %[t0], 3, %[lut]\n\t"           \
+    "ds_read_b64 v[54:55], %[t0]\n\t"
+#define VRT_LUT_MASK(lo, hi)                               \
+    "v_and_b32 v54, " lo ", v54\n\t"                       \
+    "v_and_b32 v55, " hi ", v55\n\t"
+#define VRT_LUT_TESTS                                      \
+    "v_or_b32 %[t0], v54, v55\n\t"                         \
+    "v_lshrrev_b64 v[54:55], %[t2], v[54:55]\n\t"          \
+    "v_and_b32 %[t1], 0x330033, v54\n\t"
+// VRT_STEP_SECTOR and VRT_STEP_CELL over the mask table with the ray-cell table.  A record's mask is
+// of 8- or 32-voxel cells, w = 3 or 5 their log2.
+#define VRT_LUT_SECTOR                                     \
+    VRT_STEP_RECORD("%[alive]")                            \
+    "v_lshlrev_b32 %[t2], 2, %[g2]\n\t"                    \
+    "v_lshlrev_b32 %[t1], 4, %[g1]\n\t"                    \
+    "s_waitcnt vmcnt(0)\n\t"                               \
+    "v_lshrrev_b32 %[t0], v51, %[g0]\n\t"                  \
+    "v_lshrrev_b32 %[t2], v51, %[t2]\n\t"                  \
+    "v_lshrrev_b32 %[t1], v51, %[t1]\n\t"                  \
+    "v_bitop3_b32 %[t0], 12, %[t2], %[t0] bitop3:0xca\n\t" \
+    "v_bitop3_b32 %[t1], 48, %[t1], %[t0] bitop3:0x35\n\t" \
+    VRT_LUT_READ                                           \
+    "v_bitop3_b32 %[t2], %[t1], 42, %[t1] bitop3:0x0c\n\t" \
+    "v_lshlrev_b64 v[52:53], %[t1], v[48:49]\n\t"          \
+    "v_bfm_b32 %[cm], v51, 0\n\t"                          \
+    "v_cmp_gt_i32 vcc, 0, v53\n\t"                         \
+    "s_waitcnt lgkmcnt(0)\n\t"                             \
+    VRT_LUT_MASK("v48", "v49")                             \
+    VRT_LUT_TESTS                                          \
+    "v_sub_u32 %[t0], 1, %[t0] clamp\n\t"                  \
+    "v_sub_u32 %[t1], 1, %[t1] clamp\n\t"                  \
+    "v_lshl_or_b32 %[t0], %[t0], 1, %[t1]\n\t"             \
+    "v_lshl_or_b32 %[cm], %[t0], v51, %[cm]\n\t"
+#define VRT_LUT_CELL                                       \
+    "v_lshrrev_b32 %[t2], 1, %[g2]\n\t"                    \
+    VRT_STEP_CELL_LOAD                                     \
+    VRT_LUT_READ                                           \
+    "s_waitcnt vmcnt(0)\n\t"                               \
+    "v_lshlrev_b64 v[56:57], %[t1], v[52:53]\n\t"          \
+    "v_cmp_gt_i32 vcc, 0, v57\n\t"                         \
+    "s_waitcnt lgkmcnt(0)\n\t"                             \
+    VRT_LUT_MASK("v52", "v53")                             \
+    "s_or_b64 %[stop], %[stop], vcc\n\t"                   \
+    "v_mov_b32 v52, v54\n\t"                               \
+    "v_mov_b32 v53, v55\n\t"                               \
+    VRT_LUT_TESTS
+
+// shader_loop for quick rays (ray_is_quick of the start org, d and inv): the cast's fast loop
+// (traverse.h) with this method's bias, its level above an empty sector (step records' bits 8..9) and
+// rayCastCoarse's stop in a non-empty cell from step 31 on.  The largest cell, 128 voxels, lies inside
+// the tables, so positions stay within their border as there.  A step at the sector level takes 36 vector
 // instructions (shader_loop's about 70, with no record kept between steps): 2.07 M camera rays over
 // the 1024^3 terrain 167 -> 96 us (rayCast), 80 -> 45 us (rayCastCoarse).  slot: the hit voxel's
-// brick.
-template <bool COARSE>
-__device__ __forceinline__ bool shader_loop_fast(const WorldView& w, const float d[3], const float org[3],
-                                                 const float inv[3], const float ts[3], const int32_t W[3],
+// brick.  With the ray-cell table (lut: fill_lut's result plus the ray's octant * 512) a step ands
+// the mask of its cell with the table's word, read from LDS, and a step at the sector level takes 45:
+// 0.92 M camera rays over the same terrain 69 -> 44 us (coarse), 158 -> 99 us (full).  500 k rays
+// with no order in a 64^3 world of noise, which loop up to the cap: 305 -> 181 us, 323 -> 215 with
+// the table.
+template <bool COARSE, bool LUT>
+__device__ __forceinline__ bool shader_loop_fast(const ShaderView& sv, uint32_t lut, const float d[3],
+                                                 const float org[3], const float inv[3], const float ts[3], const int32_t W[3],
                                                  const int32_t dm[3], uint32_t cap, int32_t v[3], float side[3],
                                                  float cur[3], float& tmin, uint32_t& steps, uint32_t& slot) {
+    const WorldView& w = sv.w;
     // the first step leaves the start's voxel, which may lie anywhere
 #pragma unroll
     for (int a = 0; a < 3; a++)
@@ -176,36 +242,48 @@ __device__ __forceinline__ bool shader_loop_fast(const WorldView& w, const float
     for (int a = 0; a < 3; a++) u[a] = g[a] - (0x4B000000u + (uint32_t)kStepPad);
     steps = 0;
     if (!((u[0] | u[2]) < w.size_xz && u[1] < w.size_y)) return false;
-    const i32x4 rsec = buffer_rsrc(w.steps, 16, w.step_n);
+    const i32x4 rsec = buffer_rsrc(LUT ? sv.masks : w.steps, 16, w.step_n);
     const i32x4 rocc = buffer_rsrc(w.occ - 8, 8, w.occ_n + 8u);
     uint32_t iters = cap, si = ~0u, slot1 = 0, base, it = 0;
     uint32_t cm, t0, t1, t2, mlo, mhi;
     uint64_t save, alive, stop;
-#define VRT_SHADER_STEP(bias, coarse)                                                                           \
+#define VRT_SHADER_STEP(bias, sector, cell, coarse)                                                             \
     asm volatile("s_mov_b64 %[save], exec\n\t"                                                                  \
-                 "s_branch vrt_look%=\n"                                                                        \
+                 "s_branch vrt_look%=\n\t.p2align 6\n"                                                          \
                  "vrt_advance%=:\n\t" VRT_STEP_ADVANCE("%[tm]", bias) VRT_STEP_FLOOR                            \
-                 "vrt_look%=:\n\t" VRT_STEP_SECTOR("%[alive]")                                                  \
-                 "v_lshrrev_b32 %[t0], 3, v51\n\t"                                                              \
-                 "v_and_or_b32 %[cm], %[t0], %[lod], %[cm]\n\t"                                                 \
-                 "s_cbranch_vccz vrt_advance%=\n\t" VRT_STEP_CELL coarse VRT_STEP_STOP                          \
+                 "vrt_look%=:\n\t" sector                                                                       \
+                 "s_cbranch_vccz vrt_advance%=\n\t" cell coarse VRT_STEP_STOP                                   \
                  "vrt_done%=:\n\t"                                                                              \
                  "s_mov_b64 exec, %[save]\n\t"                                                                  \
                  "v_mov_b32 %[base], v50\n\t"                                                                   \
                  "v_mov_b32 %[mlo], v52\n\t"                                                                    \
                  "v_mov_b32 %[mhi], v53"                                                                        \
                  : VRT_STEP_OUT(cur, side, g), [tm] "+&v"(tmin), [mlo] "=&v"(mlo), [mhi] "=&v"(mhi)             \
-                 : VRT_STEP_IN(org, d, inv, ts, dm, bias3, cap), [lod] "s"(0x60u)                               \
-                 : VRT_STEP_CLOBBERS)
-    if constexpr (COARSE)
-        VRT_SHADER_STEP("v_add_f32 %[tm], 0x3a83126f, %[tm]\n\t",
-                        // any voxel of the cell stops the ray once it > 30 (t0: its mask, ored)
-                        "v_cmp_ne_u32 vcc, 0, %[t0]\n\t"
-                        "s_cmp_gt_u32 %[it], 30\n\t"
-                        "s_cselect_b64 vcc, vcc, 0\n\t"
-                        "s_or_b64 %[stop], %[stop], vcc\n\t");
+                 : VRT_STEP_IN(org, d, inv, ts, dm, bias3, cap), [lod] "s"(0x60u), [lut] "v"(lut)               \
+                 : VRT_STEP_CLOBBERS, "v56", "v57", "memory")
+#define VRT_FINE "v_add_u32 %[tm], 5, %[tm]\n\t"
+#define VRT_COARSE "v_add_f32 %[tm], 0x3a83126f, %[tm]\n\t"
+// any voxel of the cell stops the ray once it > 30 (t0: its mask, ored)
+#define VRT_COARSE_STOP                 \
+    "v_cmp_ne_u32 vcc, 0, %[t0]\n\t"    \
+    "s_cmp_gt_u32 %[it], 30\n\t"        \
+    "s_cselect_b64 vcc, vcc, 0\n\t"     \
+    "s_or_b64 %[stop], %[stop], vcc\n\t"
+#define VRT_SECTOR               \
+    VRT_STEP_SECTOR("%[alive]")  \
+    "v_lshrrev_b32 %[t0], 3, v51\n\tv_and_or_b32 %[cm], %[t0], %[lod], %[cm]\n\t"
+    if constexpr (COARSE && LUT)
+        VRT_SHADER_STEP(VRT_COARSE, VRT_LUT_SECTOR, VRT_LUT_CELL, VRT_COARSE_STOP);
+    else if constexpr (COARSE)
+        VRT_SHADER_STEP(VRT_COARSE, VRT_SECTOR, VRT_STEP_CELL, VRT_COARSE_STOP);
+    else if constexpr (LUT)
+        VRT_SHADER_STEP(VRT_FINE, VRT_LUT_SECTOR, VRT_LUT_CELL, "");
     else
-        VRT_SHADER_STEP("v_add_u32 %[tm], 5, %[tm]\n\t", "");
+        VRT_SHADER_STEP(VRT_FINE, VRT_SECTOR, VRT_STEP_CELL, "");
+#undef VRT_SECTOR
+#undef VRT_COARSE_STOP
+#undef VRT_COARSE
+#undef VRT_FINE
 #undef VRT_SHADER_STEP
     const bool hit = iters < cap && (int32_t)base >= 0;
     steps = iters;
@@ -220,9 +298,9 @@ __device__ __forceinline__ bool shader_loop_fast(const WorldView& w, const float
     return hit;
 }
 
-// rayCast (COARSE = false, :162-204) or rayCastCoarse (COARSE = true, :206-243).
+// rayCast (COARSE = false, :162-204) or rayCastCoarse (COARSE = true, :206-243).  lut: fill_lut's result.
 template <bool COARSE, bool LUT>
-__device__ __forceinline__ bool shader_trace(const ShaderView& sv, const float o[3], const float d[3],
+__device__ __forceinline__ bool shader_trace(const ShaderView& sv, uint32_t lut, const float o[3], const float d[3],
                                              const int32_t W[3], uint32_t cap, ShaderHit& out) {
     const WorldView& w = sv.w;
     float start[3], org[3], inv[3], ts[3], side[3] = {0.0f, 0.0f, 0.0f}, cur[3] = {0.0f, 0.0f, 0.0f};
@@ -239,32 +317,19 @@ __device__ __forceinline__ bool shader_trace(const ShaderView& sv, const float o
     };
     float tmin = 0.0f;
     uint32_t it = 0, slot = 0;
-    bool hit, tame = true, found = false;
-    if constexpr (!LUT) {
+    bool hit;
+    const uint32_t oct = (d[0] < 0.0f ? 0u : 1u) + (d[1] < 0.0f ? 0u : 2u) + (d[2] < 0.0f ? 0u : 4u);
 #pragma unroll
-        for (int a = 0; a < 3; a++) inv[a] = reciprocal_in_range(d[a]);
-        begin();
-        // uniform: the launch's world and world origin
-        const bool fits = origin_is_guarded(W) && w.size_xz >= 128 && w.size_y >= 128;
-        if (fits && __all(ray_is_quick(org, d, inv))) {
-            hit = shader_loop_fast<COARSE>(w, d, org, inv, ts, W, dm, cap, v, side, cur, tmin, it, slot);
-            found = true;
-        }
-    }
-    if (!found) {
+    for (int a = 0; a < 3; a++) inv[a] = reciprocal_in_range(d[a]);
+    begin();
+    if (origin_is_guarded(W) && __all(ray_is_quick(org, d, inv))) {
+        hit = shader_loop_fast<COARSE, LUT>(sv, lut + oct * 512u, d, org, inv, ts, W, dm, cap, v, side, cur, tmin, it,
+                                            slot);
+    } else {
 #pragma unroll
         for (int a = 0; a < 3; a++) inv[a] = 1.0f / d[a];
         begin();
-#pragma unroll
-        for (int a = 0; a < 3; a++)
-            tame = tame && fabsf(inv[a]) < INFINITY && fabsf(ts[a]) < INFINITY && fabsf(org[a]) < 1048576.0f;
-        float len2 = d[0] * d[0] + d[1] * d[1] + d[2] * d[2];
-        tame = tame && len2 >= 0.25f && len2 <= 4.0f;
-        const uint32_t oct = (d[0] < 0.0f ? 0u : 1u) + (d[1] < 0.0f ? 0u : 2u) + (d[2] < 0.0f ? 0u : 4u);
-        if (LUT && __all(tame))
-            hit = shader_loop<COARSE, LUT, true>(sv, d, org, inv, ts, W, dm, oct, cap, v, side, cur, tmin, it);
-        else
-            hit = shader_loop<COARSE, LUT, false>(sv, d, org, inv, ts, W, dm, oct, cap, v, side, cur, tmin, it);
+        hit = shader_loop<COARSE, LUT>(sv, d, org, inv, ts, W, oct, cap, v, side, cur, tmin, it);
         if (hit) slot = brick_slot_at(w, v);
     }
     // the record is built in locals and stored once, so the result stays in registers

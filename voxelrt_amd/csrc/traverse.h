@@ -329,7 +329,8 @@ __device__ __forceinline__ uint32_t brick_slot_at(const WorldView& w, const int3
 // however few lanes are active or lines are read) and the launch for its longest waves.
 // It is written out because the compiler's loop spends 8 more scalar instructions and a branch per
 // step on lane masks for the exits (one wave alone: 183 against 162 ns per step; ray_advance's
-// loop 219).  Waits for the loads are inside the same statement.
+// loop 219).  Waits for the loads are inside the same statement.  Its start is at a 64-byte line: 0.5%
+// on the frames, 2% in the shader method.
 //
 // Quick and guarded rays.  The border is one sector wide, so no position may leave the world by 32
 // voxels or more before its lookup.  A position is o + t d with t the least of the three computed
@@ -453,8 +454,8 @@ __device__ __forceinline__ i32x4 buffer_rsrc(const void* base, uint32_t stride, 
     "s_cbranch_vccz vrt_advance%=\n\t"                         \
     "s_mov_b64 exec, vcc\n\t"
 // The sector record, loaded by the lanes that have entered another sector (lanes: what to save
-// exec in), then the brick's mask bit (v53's sign) and the sector-level cell mask.
-#define VRT_STEP_SECTOR(lanes)                                 \
+// exec in).
+#define VRT_STEP_RECORD(lanes)                                 \
     "v_bfe_u32 %[t0], %[g0], 5, 15\n\t"                        \
     "v_bfe_u32 %[t1], %[g1], 5, 15\n\t"                        \
     "v_bfe_u32 %[t2], %[g2], 5, 15\n\t"                        \
@@ -466,7 +467,9 @@ __device__ __forceinline__ i32x4 buffer_rsrc(const void* base, uint32_t stride, 
     "buffer_load_dwordx4 v[48:51], %[t1], %[rsec], 0 idxen\n\t" \
     "v_mov_b32 %[si], %[t1]\n"                                 \
     "vrt_kept%=:\n\t"                                          \
-    "s_mov_b64 exec, " lanes "\n\t"                            \
+    "s_mov_b64 exec, " lanes "\n\t"
+// The record, then the brick's mask bit (v53's sign) and the sector-level cell mask.
+#define VRT_STEP_SECTOR(lanes) VRT_STEP_RECORD(lanes)          \
     "v_lshrrev_b32 %[t2], 1, %[g2]\n\t"                        \
     "v_lshrrev_b32 %[t0], 3, %[g0]\n\t"                        \
     "v_lshlrev_b32 %[t1], 1, %[g1]\n\t"                        \
@@ -480,9 +483,9 @@ __device__ __forceinline__ i32x4 buffer_rsrc(const void* base, uint32_t stride, 
     "v_lshrrev_b32 %[t0], %[t0], v51\n\t"                      \
     "v_bitop3_b32 %[cm], %[t0], 24, 7 bitop3:0xea\n\t"
 // Lanes vcc are in an allocated brick or outside the world (the border's base slot is negative).
-// The first look their 4x4x4 cell's mask up (v[52:53]; slot: their brick's slot + 1), and stop at
-// a solid voxel; t1 and t2 are the voxel's shifts.
-#define VRT_STEP_CELL                                          \
+// The first look their 4x4x4 cell's mask up (v[52:53]; slot: their brick's slot + 1); t1 and t2
+// are the voxel's shifts.  t2 is g2 >> 1 before.
+#define VRT_STEP_CELL_LOAD                                     \
     "s_mov_b64 exec, vcc\n\t"                                  \
     "v_cmp_gt_i32 vcc, 0, v50\n\t"                             \
     "s_mov_b64 %[stop], vcc\n\t"                               \
@@ -501,7 +504,9 @@ __device__ __forceinline__ i32x4 buffer_rsrc(const void* base, uint32_t stride, 
     "v_lshlrev_b32 %[t1], 4, %[g1]\n\t"                        \
     "v_bitop3_b32 %[t2], 12, %[t2], %[g0] bitop3:0xca\n\t"     \
     "v_bitop3_b32 %[t1], 48, %[t1], %[t2] bitop3:0x35\n\t"     \
-    "v_bitop3_b32 %[t2], %[t1], 42, %[t1] bitop3:0x0c\n\t"     \
+    "v_bitop3_b32 %[t2], %[t1], 42, %[t1] bitop3:0x0c\n\t"
+// Then they stop at a solid voxel.
+#define VRT_STEP_CELL VRT_STEP_CELL_LOAD                       \
     "s_waitcnt vmcnt(0)\n\t"                                   \
     "v_lshlrev_b64 v[54:55], %[t1], v[52:53]\n\t"              \
     "v_or_b32 %[t0], v52, v53\n\t"                             \
@@ -566,7 +571,7 @@ __device__ __forceinline__ bool ray_trace_fast(const WorldView& w, RayState& r, 
         uint32_t gi = ~0u;
         uint64_t lanes;
         asm volatile("s_mov_b64 %[save], exec\n\t"
-                     "s_branch vrt_look%=\n"
+                     "s_branch vrt_look%=\n\t.p2align 6\n"
                      "vrt_back%=:\n\t"
                      "s_mov_b64 exec, %[alive]\n"
                      "vrt_advance%=:\n\t" VRT_STEP_ADVANCE("%[t0]", VRT_STEP_BIAS)
@@ -580,7 +585,7 @@ __device__ __forceinline__ bool ray_trace_fast(const WorldView& w, RayState& r, 
                      : VRT_STEP_CLOBBERS, "v56", "v57");
     } else {
         asm volatile("s_mov_b64 %[save], exec\n\t"
-                     "s_branch vrt_look%=\n"
+                     "s_branch vrt_look%=\n\t.p2align 6\n"
                      "vrt_advance%=:\n\t" VRT_STEP_ADVANCE("%[t0]", VRT_STEP_BIAS)
                      VRT_STEP_FLOOR "vrt_look%=:\n\t" VRT_STEP_SECTOR("%[alive]")
                      "s_cbranch_vccz vrt_advance%=\n\t" VRT_STEP_BRICK

@@ -92,7 +92,9 @@ constexpr int32_t kStepPad = 128;
 // The group table: per group of 4x4x4 sectors a u64, bit x | z << 2 | y << 4 set when that sector
 // has a brick or lies outside the world.  Group (X, Y, Z) of the padded coordinates (>> 7) is word
 // X + Z * group_z + Y * group_y.
-// The step table: per sector and for the border of one sector around the world a 16-byte record.
+// The step table: per sector a 16-byte record, and border records around them: one sector before the
+// world, and after it up to one past the world's last sector or the group of 4, whichever is
+// further (the shader method's cells are up to a group wide).
 // Sector (X, Y, Z) of the padded coordinates (>> 5; the world's first is 4, the border's 3) is
 // record X + Z * step_z + Y * step_y; the records before the border's first are never read.
 //   x, y  allocation mask; all ones in the border (the step's brick test then succeeds)
@@ -119,6 +121,15 @@ __host__ __device__ inline uint32_t group_lod(uint64_t group, uint32_t sector) {
     const uint32_t half = sector < 32 ? (uint32_t)group : (uint32_t)(group >> 32);
     return group == 0 ? 3u : (((half >> (sector & 0xAu)) & 0x00330033u) == 0 ? 1u : 0u);
 }
+// The mask table: the step table's records by index, as the ray-cell table (ShaderView) needs them.
+//   x, y  allocation mask; of an empty sector its group's mask, in which its own bit is 0, so
+//         the step's brick test fails there too; all ones in the border
+//   z     base slot; all ones in the border
+//   w     log2 of the voxels per bit of that mask: 3, or 5 for an empty sector
+__host__ __device__ inline uint4 mask_record(uint64_t mask, uint32_t base, uint64_t group) {
+    const uint64_t m = mask ? mask : group;
+    return make_uint4((uint32_t)m, (uint32_t)(m >> 32), base, mask ? 3u : 5u);
+}
 inline __host__ __device__ uint4 step_border_record() { return make_uint4(~0u, ~0u, ~0u, 0u); }
 
 struct WorldView {
@@ -140,6 +151,7 @@ struct WorldView {
 struct ShaderView {
     WorldView w;
     const uint64_t* __restrict__ groups;  // [1 << (2 * gshift_xz + gshift_y)]
+    const uint4* __restrict__ masks;      // [w.step_n] the mask table
     const uint64_t* __restrict__ lut;     // [8 octants * 64 cells]
     uint32_t gshift_xz, gshift_y;
 };
@@ -159,6 +171,7 @@ struct vrt_world {
     uint8_t* d_tables = nullptr;      // one allocation for every table but d_occ and d_vox
     uint4* d_sec = nullptr;           // packed sector records (mask, base slot)
     uint4* d_steps = nullptr;         // the step table
+    uint4* d_masks = nullptr;         // the mask table
     uint64_t* d_sgroups = nullptr;    // the group table
     uint64_t* d_occ = nullptr;
     uint8_t* d_vox = nullptr;
@@ -199,10 +212,11 @@ struct vrt_world {
     // totals since creation
     uint64_t upload_bytes = 0, upload_brick_bytes = 0, moved_bricks = 0;
 
-    uint32_t step_z() const { return (1u << shift_xz) + 2u; }
+    // at least 4 sectors a side and the border
+    uint32_t step_z() const { return std::max(4u, 1u << shift_xz) + 2u; }
     uint32_t step_y() const { return step_z() * step_z(); }
     uint32_t step_first() const { return 3u + 3u * step_z() + 3u * step_y(); }
-    uint32_t step_n() const { return step_first() + step_y() * ((1u << shift_y) + 2u); }
+    uint32_t step_n() const { return step_first() + step_y() * (std::max(4u, 1u << shift_y) + 2u); }
     uint32_t group_z() const { return (1u << gshift_xz) + 2u; }
     uint32_t group_y() const { return group_z() * group_z(); }
     uint32_t group_n() const { return group_y() * ((1u << gshift_y) + 2u); }
@@ -238,6 +252,7 @@ struct vrt_world {
         vrt::ShaderView v;
         v.w = view();
         v.groups = d_groups;
+        v.masks = d_masks;
         v.lut = d_lut;
         v.gshift_xz = gshift_xz;
         v.gshift_y = gshift_y;

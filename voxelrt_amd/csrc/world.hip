@@ -179,21 +179,22 @@ __global__ __launch_bounds__(256) void sync_place_kernel(uint8_t* __restrict__ v
 // The tables of an empty world: records of empty sectors, in the step and group tables with a border
 // around them, no group bits and a zero palette.
 struct WorldTables {
-    uint4 *sec, *steps;
+    uint4 *sec, *steps, *masks;
     uint64_t *groups, *sgroups, *palette;
-    uint32_t nsec, step_z, step_y, step_first, step_n, ngroups, group_z, group_y, group_n;
+    uint32_t nsec, step_z, step_y, step_first, step_n, nxz, ny, ngroups, group_z, group_y, group_n;
     uint64_t outside;
 };
 __global__ __launch_bounds__(256) void world_init_kernel(WorldTables t) {
     const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i < t.nsec) t.sec[i] = sector_record(0, 0);
     if (i < t.step_n) {
-        const uint32_t k = i < t.step_first ? 0u : i - t.step_first, ny = (t.step_n - t.step_first) / t.step_y;
+        const uint32_t k = i < t.step_first ? 0u : i - t.step_first;
         const uint32_t y = k / t.step_y, z = k % t.step_y / t.step_z, x = k % t.step_z;
-        const bool border = x == 0 || x == t.step_z - 1 || z == 0 || z == t.step_z - 1 || y == 0 || y == ny - 1;
+        const bool border = x == 0 || x > t.nxz || z == 0 || z > t.nxz || y == 0 || y > t.ny;
         uint4 r = border ? step_border_record() : step_record(0, 0);
         if (!border) r.w |= group_lod(0, 0) << 8;
         t.steps[i] = r;
+        t.masks[i] = border ? r : mask_record(0, 0, 0);
     }
     if (i < t.ngroups) t.groups[i] = 0;
     if (i < t.group_n) {
@@ -205,9 +206,9 @@ __global__ __launch_bounds__(256) void world_init_kernel(WorldTables t) {
     if (i < 256) t.palette[i] = 0;
 }
 
-// Records of the synced sectors (indices unique), in both tables.
+// Records of the synced sectors (indices unique), in all three tables.
 struct StepTables {
-    uint4* steps;
+    uint4 *steps, *masks;
     uint64_t* groups;
     uint32_t shift_xz, gshift_xz, step_z, step_y, group_z, group_y;
     uint64_t outside;  // bits of a group word outside the world
@@ -221,12 +222,14 @@ __global__ __launch_bounds__(256) void sync_records_kernel(uint4* __restrict__ s
         const uint4 r = rec[i];
         sec[s] = r;
         const uint32_t X = (s & n1) + 4u, Z = ((s >> st.shift_xz) & n1) + 4u, Y = (s >> (2 * st.shift_xz)) + 4u;
-        st.steps[X + Z * st.step_z + Y * st.step_y] = step_record((uint64_t)r.x | (uint64_t)r.y << 32, r.z);
+        const uint64_t m = (uint64_t)r.x | (uint64_t)r.y << 32;
+        st.steps[X + Z * st.step_z + Y * st.step_y] = step_record(m, r.z);
+        st.masks[X + Z * st.step_z + Y * st.step_y] = mask_record(m, r.z, 0);
     }
 }
 
 // Changed sector-of-sectors words, thread (word, sector of it): the word goes to both tables, and
-// the empty sectors' step records get their level above the sector.  After the records.
+// the empty sectors' step and mask records get the level above the sector.  After the records.
 __global__ __launch_bounds__(256) void sync_groups_kernel(StepTables st, uint64_t* __restrict__ groups,
                                                           const uint64_t* __restrict__ gval,
                                                           const uint32_t* __restrict__ gidx, uint32_t ngrp) {
@@ -244,6 +247,7 @@ __global__ __launch_bounds__(256) void sync_groups_kernel(StepTables st, uint64_
     uint4 r = step_record(0, 0);
     r.w |= group_lod(m, b) << 8;
     st.steps[X + Z * st.step_z + Y * st.step_y] = r;
+    st.masks[X + Z * st.step_z + Y * st.step_y] = mask_record(0, 0, m);
 }
 
 }  // namespace vrt
@@ -569,7 +573,7 @@ static int world_sync(vrt_world* w, uint32_t nsec, const uint32_t* sector_idx, c
         gval.push_back(v);
     }
     const uint64_t nrec = nsec, ngrp = gidx.size();
-    const StepTables st{w->d_steps, w->d_sgroups, w->shift_xz, w->gshift_xz, w->step_z(), w->step_y(),
+    const StepTables st{w->d_steps, w->d_masks, w->d_sgroups, w->shift_xz, w->gshift_xz, w->step_z(), w->step_y(),
                         w->group_z(), w->group_y(), w->group_outside()};
     for (uint64_t r0 = 0, g0 = 0; r0 < nrec || g0 < ngrp;) {
         uint32_t nr = (uint32_t)std::min<uint64_t>(nrec - r0, (kSyncHalf - 256) / 20);
@@ -673,6 +677,7 @@ int vrt_world_create(const vrt_world_desc* desc, void* stream, vrt_world** out) 
             return at;
         };
         const size_t o_sec = part((size_t)w->nsec * 16), o_steps = part((size_t)w->step_n() * 16);
+        const size_t o_masks = part((size_t)w->step_n() * 16);
         const size_t o_groups = part(w->h_groups.size() * 8), o_sgroups = part((size_t)w->group_n() * 8);
         const size_t o_palette = part(256 * 8), o_lut = part(512 * 8);
         check(hipMalloc(&w->d_tables, bytes), "hipMalloc(world tables)");
@@ -681,14 +686,15 @@ int vrt_world_create(const vrt_world_desc* desc, void* stream, vrt_world** out) 
             std::memset(w->h_pick, 0, kPickBytes);
             w->d_sec = (uint4*)(w->d_tables + o_sec);
             w->d_steps = (uint4*)(w->d_tables + o_steps);
+            w->d_masks = (uint4*)(w->d_tables + o_masks);
             w->d_groups = (uint64_t*)(w->d_tables + o_groups);
             w->d_sgroups = (uint64_t*)(w->d_tables + o_sgroups);
             w->d_palette = (uint64_t*)(w->d_tables + o_palette);
             w->d_lut = (uint64_t*)(w->d_tables + o_lut);
-            const WorldTables t{w->d_sec,       w->d_steps,     w->d_groups, w->d_sgroups, w->d_palette,
+            const WorldTables t{w->d_sec,       w->d_steps,     w->d_masks, w->d_groups, w->d_sgroups, w->d_palette,
                                 w->nsec,        w->step_z(),    w->step_y(), w->step_first(), w->step_n(),
-                                (uint32_t)w->h_groups.size(),   w->group_z(), w->group_y(), w->group_n(),
-                                w->group_outside()};
+                                1u << w->shift_xz, 1u << w->shift_y, (uint32_t)w->h_groups.size(),
+                                w->group_z(),   w->group_y(),   w->group_n(), w->group_outside()};
             const uint32_t n = std::max({w->nsec, w->step_n(), w->group_n(), 256u});
             world_init_kernel<<<(n + 255) / 256, 256, 0, s>>>(t);
             check(hipGetLastError(), "world_init_kernel");
@@ -724,9 +730,9 @@ int vrt_world_get_info(const vrt_world* w, vrt_world_info* out) {
         out->num_sectors = w->nsec;
         out->num_bricks = w->num_bricks;
         out->slot_capacity = w->slot_cap;
-        out->device_bytes = (uint64_t)w->nsec * 16 + (uint64_t)w->step_n() * 16 + (uint64_t)w->group_n() * 8 + 256 * 8 + (uint64_t)w->slot_cap * (512 + 64) +
-                            (uint64_t)w->h_groups.size() * 8 + 512 * 8 + (w->d_stage ? 2 * kSyncHalf : 0) +
-                            w->moves_cap;
+        out->device_bytes = (uint64_t)w->nsec * 16 + (uint64_t)w->step_n() * 32 + (uint64_t)w->group_n() * 8 +
+                            256 * 8 + (uint64_t)w->slot_cap * (512 + 64) + (uint64_t)w->h_groups.size() * 8 +
+                            512 * 8 + (w->d_stage ? 2 * kSyncHalf : 0) + w->moves_cap;
         out->slot_high_water = w->arena.high_water();
         out->generation = w->generation;
         out->upload_bytes = w->upload_bytes;
