@@ -195,11 +195,14 @@ __device__ __forceinline__ void trace_block(const WorldView& w, const BatchArgs&
     }
 }
 
-// One wave per block of the virtual index space; the hardware dispatcher balances waves.
+// One wave per block of the virtual index space; the hardware dispatcher balances waves.  The last
+// block goes first: a camera's cheap top rows, and the cameras before the ray sets that follow
+// them, then run in the launch's tail (24 cameras with 8 ray sets: 512 -> 495 us).
 template <int RPL, bool COUNT>
 __global__ __launch_bounds__(256) void batch_grid_kernel(WorldView w, BatchArgs a, vrt_cast_counters* ctr) {
     uint32_t block = blockIdx.x * (blockDim.x / 64) + threadIdx.x / 64;
     if (block >= a.nblocks) return;  // wave-uniform
+    block = a.nblocks - 1u - xcd_window_block(block, a.nblocks);
     trace_block<RPL, COUNT>(w, a, block, ctr);
 }
 

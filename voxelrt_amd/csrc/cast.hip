@@ -93,11 +93,13 @@ constexpr uint32_t kGridThreads = 64;
 // chip drains.  A camera's last rows (the ground, with descents and hits) cost the
 // most per wave and its first rows (sky) the least, so the reverse order leaves cheap
 // waves for the tail: 0.118 against 0.139 ms for the 1920x1080 primary rays.  A random
-// block order (0.145 ms) loses the L2 reuse between neighbouring tiles.
+// block order (0.145 ms) loses the L2 reuse between neighbouring tiles; in a window of 512
+// blocks each XCD takes neighbours (xcd_window_block).
 template <bool COUNT, bool GROUPS>
 __global__ __launch_bounds__(kGridThreads) void cast_grid_kernel(WorldView w, RaysIn r, HitsOut h, uint32_t max_iters,
                                                                  vrt_cast_counters* ctr, uint32_t reverse) {
-    uint32_t blk = reverse ? gridDim.x - 1u - blockIdx.x : blockIdx.x;
+    uint32_t blk = xcd_window_block(blockIdx.x, gridDim.x);
+    if (reverse) blk = gridDim.x - 1u - blk;
     uint32_t i = blk * kGridThreads + threadIdx.x;
     bool valid = i < ray_count(r);
     RayState st;

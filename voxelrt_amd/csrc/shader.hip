@@ -12,7 +12,7 @@ namespace {
 
 template <bool COARSE, bool LUT>
 __global__ __launch_bounds__(256) void shader_cast_kernel(ShaderView sv, RaysIn r, HitsOut h, uint32_t cap) {
-    uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
+    uint32_t i = xcd_window_block(blockIdx.x, gridDim.x) * blockDim.x + threadIdx.x;
     __shared__ uint4 lds_lut[LUT ? kLutPairs : 1];
     const uint32_t lut = fill_lut<LUT>(sv, lds_lut);
     if (i >= r.n) return;

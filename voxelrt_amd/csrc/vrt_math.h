@@ -135,6 +135,18 @@ __host__ __device__ inline void tile_pixel(uint32_t i, const tile_map& m, uint32
     py = ty * m.tile_h + row;
 }
 
+// The b-th dispatched block's place among n.  Block b runs on XCD b % 8; of every 512 blocks each
+// XCD here takes 64 neighbours, so that their rays meet in its L2, and windows of 512 differ too
+// little in work to leave an XCD behind.  One 1024x576 camera with positions 52.4 -> 47.9 us, 24
+// cameras with 8 ray sets 495 -> 482 (runs of 8 487, of 256 477), 1920x1080 primary and bounce rays
+// 158.5 -> 156.8.  The fused frame, the G-buffer and the differentiable forward gain nothing and
+// keep their order.
+constexpr uint32_t kXcdRun = 64;
+__host__ __device__ inline uint32_t xcd_window_block(uint32_t b, uint32_t n) {
+    const uint32_t q = b / (8 * kXcdRun), r = b % (8 * kXcdRun);
+    return q < n / (8 * kXcdRun) ? q * (8 * kXcdRun) + r % 8 * kXcdRun + r / 8 : b;
+}
+
 // normalize(N + s) for s uniform on the unit sphere from the next two PCG
 // samples of st (random_dir, RandomGen.glsl:37-48, with PCG samples in place of
 // the blue-noise texture); N + s = 0 falls back to N.
