@@ -146,7 +146,7 @@ __global__ __launch_bounds__(256) void render_bwd_kernel(uint32_t n, const float
 // float atomics.  The other entries are zeros, and they are most of it: 16 views of 512 x 512 over the
 // 512^3 terrain touch 8.9 k of its 97 k slots (1.7 M pixels, 195 per touched slot).  So the gradient is
 // filled with zeros first, at the rate of a fill, and the touched slots are written a second time.
-// Measured there (598 MB), in us: fill 77, counts 33, allocation 5, placement 24, sums 19, against 197
+// Measured there (598 MB), in us: fill 77, counts 27, allocation 5, placement 24, sums 19, against 197
 // for six launches the last of which wrote each slot's zeros or sums by a wave.  Sharing a launch
 // between the fill and the counts or the placement gained nothing (they wait for each other's memory),
 // nor did filling after the placement (counts and placement 8 faster, sums 5 slower, a launch more).
@@ -167,61 +167,74 @@ __global__ __launch_bounds__(256) void bwd_fill_kernel(float4* __restrict__ out,
 }
 
 // Pass 1: the rank of each contributing pixel among the pixels of its slot; counts[slot] ends
-// as the slot's pixel count.  Lanes of a wave with the same slot share one atomic (each round
-// matches the first pending lane's slot by ballot; a lane's rank is its position among the
-// matches).  Eight rounds, unrolled with one result variable each, so a wave's atomics are all
-// in flight together and the wave waits for their returns once, after the last round.  Bound by the
-// atomics, which are performed past the XCDs' L2s, 23 to an address here: with four rows of pixels in
-// flight per wave it took 42 us and not 30.
-__global__ __launch_bounds__(256) void bwd_count_kernel(uint32_t n, const uint32_t* __restrict__ saved_voxel,
-                                                        const float* __restrict__ saved_weight,
-                                                        uint32_t* __restrict__ counts, uint32_t* __restrict__ rank) {
-    uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-    uint32_t slot = 0xFFFFFFFFu;
-    if (i < n) {
-        uint32_t gv = saved_voxel[i];
-        if (gv != 0xFFFFFFFFu && saved_weight[i] != 0.0f) slot = gv >> 9;
+// as the slot's pixel count.  Lanes of a wave with the same slot are matched by ballot (eight
+// rounds, each for the first pending lane's slot; a lane left over stands for itself), the block's
+// slots meet in an LDS table, and each slot in it takes its room with one global atomic.  The
+// atomics are performed past the XCDs' L2s and serialize on a slot that fills much of an image: one per
+// wave and slot took 33 us for the 16 views and 12.7 for three of 375x281, one per block 26.8 and 7.9
+// (blocks of 512 and 1024 pixels 27-30 and 6.2-10).
+constexpr uint32_t kCountThreads = 256;
+constexpr uint32_t kCountTable = 2 * kCountThreads;  // never more than half full
+__global__ __launch_bounds__(kCountThreads) void bwd_count_kernel(uint32_t n, const uint32_t* __restrict__ saved_voxel,
+                                                                  const float* __restrict__ saved_weight,
+                                                                  uint32_t* __restrict__ counts,
+                                                                  uint32_t* __restrict__ rank) {
+    __shared__ uint32_t keys[kCountTable], cnt[kCountTable];
+    const uint32_t t = threadIdx.x, lane = __lane_id();
+    const uint32_t i = blockIdx.x * kCountThreads + t;
+    const uint32_t gv = i < n ? saved_voxel[i] : 0xFFFFFFFFu;
+    const float weight = i < n ? saved_weight[i] : 0.0f;
+#pragma unroll
+    for (uint32_t k = t; k < kCountTable; k += kCountThreads) {
+        keys[k] = 0xFFFFFFFFu;
+        cnt[k] = 0u;
     }
-    bool pending = slot != 0xFFFFFFFFu;
-    const uint32_t lane = __lane_id();
-    uint32_t my_leader = 0;
-    uint64_t my_same = 0;
-    bool matched = false;
-    // one round: the leader's atomic result lands in its own variable b, read only after the
-    // last round
-    auto round = [&](uint32_t& b) {
-        uint64_t todo = __ballot(pending);
-        if (todo == 0) return;  // wave-uniform
-        uint32_t leader = (uint32_t)__ffsll((unsigned long long)todo) - 1u;
-        uint32_t key = __shfl(slot, (int)leader, 64);
-        bool mine = pending && slot == key;
-        uint64_t same = __ballot(mine);
-        if (lane == leader) b = atomicAdd(&counts[key], (uint32_t)__popcll(same));
+    __syncthreads();
+    const bool in = gv != 0xFFFFFFFFu && weight != 0.0f;
+    const uint32_t slot = gv >> 9;  // below 2^23
+    bool pending = in;
+    uint32_t leader = lane;
+    uint64_t same = 1ull << lane;
+#pragma unroll 1
+    for (int k = 0; k < 8; k++) {
+        const uint64_t todo = __ballot(pending);
+        if (todo == 0) break;  // wave-uniform
+        const uint32_t first = (uint32_t)__builtin_ctzll(todo);
+        const uint32_t key = __builtin_amdgcn_readlane(slot, first);
+        const bool mine = pending && slot == key;
+        const uint64_t m = __ballot(mine);
         if (mine) {
-            my_leader = leader;
-            my_same = same;
-            matched = true;
+            leader = first;
+            same = m;
             pending = false;
         }
-    };
-    uint32_t b0 = 0, b1 = 0, b2 = 0, b3 = 0, b4 = 0, b5 = 0, b6 = 0, b7 = 0;
-    round(b0);
-    round(b1);
-    round(b2);
-    round(b3);
-    round(b4);
-    round(b5);
-    round(b6);
-    round(b7);
-    // a lane leads at most one round and its other variables stay 0, so their OR is the base of
-    // the round it led
-    uint32_t led = b0 | b1 | b2 | b3 | b4 | b5 | b6 | b7;
-    uint32_t r = 0xFFFFFFFFu;
-    uint32_t b = __shfl(led, (int)my_leader, 64);
-    if (matched)
-        r = b + __builtin_amdgcn_mbcnt_hi((uint32_t)(my_same >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)my_same, 0u));
-    if (pending) r = atomicAdd(&counts[slot], 1u);  // slots left after the unrolled rounds
-    if (i < n) rank[i] = r;
+    }
+    // the leaders find their slot's entry: at most 256 of 512 are taken, so a free one ends the search
+    uint32_t h = 0, base = 0;
+    if (in && leader == lane) {
+        h = (slot * 2654435761u) >> (32 - __builtin_ctz(kCountTable));
+        for (;;) {
+            const uint32_t k = atomicCAS(&keys[h], 0xFFFFFFFFu, slot);
+            if (k == 0xFFFFFFFFu || k == slot) break;
+            h = (h + 1) & (kCountTable - 1u);
+        }
+        base = atomicAdd(&cnt[h], (uint32_t)__popcll(same));
+    }
+    __syncthreads();
+    uint32_t from[2];
+#pragma unroll
+    for (uint32_t p = 0; p < 2; p++) {
+        const uint32_t k = keys[t + p * kCountThreads];
+        from[p] = k != 0xFFFFFFFFu ? atomicAdd(&counts[k], cnt[t + p * kCountThreads]) : 0u;
+    }
+#pragma unroll
+    for (uint32_t p = 0; p < 2; p++) cnt[t + p * kCountThreads] = from[p];
+    __syncthreads();
+    if (in && leader == lane) base += cnt[h];
+    base = __shfl(base, (int)leader, 64);
+    const uint32_t before =
+        __builtin_amdgcn_mbcnt_hi((uint32_t)(same >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)same, 0u));
+    if (i < n) rank[i] = in ? base + before : 0xFFFFFFFFu;
 }
 
 // Pass 2: the slots' lists and the list of the touched slots.  A block scans kScanBlock counts
@@ -496,7 +509,8 @@ int vrt_render_bwd_bricks(const vrt_world* world, uint32_t npixels, const float*
         bwd_fill_kernel<<<(uint32_t)((vecs + tail + words + 255) / 256), 256, 0, s>>>((float4*)grad_albedo, vecs, tail,
                                                                                      ws.cursor, words);
         if (npixels) {
-            bwd_count_kernel<<<(npixels + 255) / 256, 256, 0, s>>>(npixels, saved_voxel, saved_weight, ws.counts, ws.rank);
+            bwd_count_kernel<<<(npixels + kCountThreads - 1) / kCountThreads, kCountThreads, 0, s>>>(
+                npixels, saved_voxel, saved_weight, ws.counts, ws.rank);
             bwd_alloc_kernel<<<nblk, 256, 0, s>>>(ns, ws.counts, ws.cursor, ws.offsets, ws.touched);
             bwd_place_kernel<<<(npixels + 255) / 256, 256, 0, s>>>(npixels, grad_image, saved_voxel, saved_weight, ws.rank,
                                                                    ws.offsets, ws.list);
