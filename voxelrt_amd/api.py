@@ -23,11 +23,23 @@ from . import _lib as L
 
 def _stream_handle(stream) -> int | None:
     if stream is None:
-        # torch's current stream; the null stream when torch sees no device (the library reports the error)
-        return torch.cuda.current_stream().cuda_stream if torch.cuda.is_available() else 0
+        # torch's current stream; the null stream when torch sees no device (the library reports the error).
+        # Its handle alone: a Stream object around it took 2.7 us of a launch's 18, this 0.3
+        if not torch.cuda.is_available():
+            return 0
+        return torch._C._cuda_getCurrentRawStream(torch.cuda.current_device())
     if isinstance(stream, torch.cuda.Stream):
         return stream.cuda_stream
     return int(stream)
+
+
+def _rows3(t: torch.Tensor) -> tuple:
+    """Pointers to t[0], t[1] and t[2], without the three views (1 us each)."""
+    if t.shape[0] < 3:
+        raise IndexError(f"index 2 is out of bounds for dimension 0 with size {t.shape[0]}")
+    p = t.data_ptr()
+    s = t.stride(0) * t.element_size() if p else 0  # no elements, no memory
+    return p, p + s, p + 2 * s
 
 
 def _ptr(t) -> int:
@@ -196,10 +208,7 @@ class RayBatch:
         return int(self.o.shape[1])
 
     def to_c(self) -> L.Rays:
-        o, d = self.o, self.d
-        r = L.Rays(o[0].data_ptr(), o[1].data_ptr(), o[2].data_ptr(), d[0].data_ptr(), d[1].data_ptr(),
-                   d[2].data_ptr(), (C.c_int32 * 3)(*self.world_origin), self.n)
-        return r
+        return L.Rays(*_rows3(self.o), *_rows3(self.d), (C.c_int32 * 3)(*self.world_origin), self.n)
 
     @staticmethod
     def from_numpy(o: np.ndarray, d: np.ndarray, world_origin=(0, 0, 0), device="cuda") -> "RayBatch":
@@ -214,9 +223,7 @@ class RayBatch:
                         tuple(int(x) for x in world_origin))
 
     def buffers(self) -> L.RayBuffers:
-        o, d = self.o, self.d
-        return L.RayBuffers(o[0].data_ptr(), o[1].data_ptr(), o[2].data_ptr(), d[0].data_ptr(), d[1].data_ptr(),
-                            d[2].data_ptr())
+        return L.RayBuffers(*_rows3(self.o), *_rows3(self.d))
 
 
 @dataclass
@@ -491,7 +498,7 @@ def bounce(rays: RayBatch, hits: HitBatch, width: int, seed: int, stream=None, o
     dev = rays.o.device
     out = RayBatch.empty(n, rays.world_origin, dev)
     src = torch.empty(n, dtype=torch.int32, device=dev)
-    count = torch.zeros(1, dtype=torch.int32, device=dev)
+    count = torch.empty(1, dtype=torch.int32, device=dev)  # written by every generation, of no rays too
     scratch = torch.empty(int(L.lib().vrt_bounce_scratch_bytes(n)) // 4 + 1, dtype=torch.int32, device=dev)
     r = rays.to_c()
     h = hits.to_c()
