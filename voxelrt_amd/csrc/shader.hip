@@ -12,7 +12,9 @@ namespace {
 
 template <bool COARSE, bool LUT>
 __global__ __launch_bounds__(256) void shader_cast_kernel(ShaderView sv, RaysIn r, HitsOut h, uint32_t cap) {
-    uint32_t i = xcd_window_block(blockIdx.x, gridDim.x) * blockDim.x + threadIdx.x;
+    // last block first: a camera's cheap top rows run in the launch's tail.  1280x720 over the 1024^3
+    // terrain: coarse with the table 43.1 -> 40.0 us, full 95.2 -> 91.4; 1920x1080 full 93.3 -> 90.3
+    uint32_t i = (gridDim.x - 1u - xcd_window_block(blockIdx.x, gridDim.x)) * blockDim.x + threadIdx.x;
     __shared__ uint4 lds_lut[LUT ? kLutPairs : 1];
     const uint32_t lut = fill_lut<LUT>(sv, lds_lut);
     if (i >= r.n) return;
