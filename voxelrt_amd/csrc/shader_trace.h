@@ -210,11 +210,11 @@ __device__ __forceinline__ uint32_t fill_lut(const ShaderView& sv, uint4* lut) {
 // shader_loop for quick rays (ray_is_quick of the start org, d and inv): the cast's fast loop
 // (traverse.h) with this method's bias, its level above an empty sector (step records' bits 8..9) and
 // rayCastCoarse's stop in a non-empty cell from step 31 on.  The largest cell, 128 voxels, lies inside
-// the tables, so positions stay within their border as there.  A step at the sector level takes 36 vector
+// the tables, so positions stay within their border as there.  A step at the sector level takes 37 vector
 // instructions (shader_loop's about 70, with no record kept between steps): 2.07 M camera rays over
 // the 1024^3 terrain 167 -> 96 us (rayCast), 80 -> 45 us (rayCastCoarse).  slot: the hit voxel's
 // brick.  With the ray-cell table (lut: fill_lut's result plus the ray's octant * 512) a step ands
-// the mask of its cell with the table's word, read from LDS, and a step at the sector level takes 45:
+// the mask of its cell with the table's word, read from LDS, and a step at the sector level takes 46:
 // 0.92 M camera rays over the same terrain 69 -> 44 us (coarse), 158 -> 99 us (full).  500 k rays
 // with no order in a 64^3 world of noise, which loop up to the cap: 305 -> 181 us, 323 -> 215 with
 // the table.

@@ -312,8 +312,8 @@ __device__ __forceinline__ uint32_t brick_slot_at(const WorldView& w, const int3
 // operands (f32 add, multiply and fma, and / or / xor, right shifts, adds, V_BITOP3_B32), and in 4
 // when it is another (conversions, compares, minima, bitfield inserts and extracts, left and 64-bit
 // shifts, V_OR3 and the like) or reads a scalar register.  Both kinds measured with 8 waves per
-// SIMD: 2.1-2.5 and 4.1-4.3 cycles.  A step that stays at the sector level takes 34 vector
-// instructions, 10 of them of the slow kind, and 9 scalar ones and branches (ray_advance: 47, 27
+// SIMD: 2.1-2.5 and 4.1-4.3 cycles.  A step that stays at the sector level takes 35 vector
+// instructions, 7 of them of the slow kind, and 9 scalar ones and branches (ray_advance: 47, 27
 // and 23):
 //   position     g = position + bias rounded down, bias = 2^23 + W + kStepPad: the bits of g are
 //                2^23's with the padded voxel coordinate in the mantissa, so one addition in the
@@ -396,6 +396,14 @@ __device__ __forceinline__ i32x4 buffer_rsrc(const void* base, uint32_t stride, 
     return r;
 }
 
+// What the record's index is too large by with the coordinates' exponent bits left in: 2^23's bits
+// >> 5, of which the products take the low 24.  Negated.  (Taking them out of each coordinate is
+// three bitfield extracts of 4 cycles for three shifts of 2 and an addition: 0.6% on the frames.)
+__device__ __forceinline__ uint32_t step_bias(const WorldView& w) {
+    constexpr uint32_t e = 0x4B000000u >> 5, e24 = e & 0xFFFFFFu;
+    return 0u - (e + e24 * w.step_z + e24 * w.step_y);
+}
+
 // The parts of the fast loop (operands: ray_trace_fast).  Fixed registers: v[48:51] the kept
 // sector record, v[52:55] temporaries, v[56:57] the kept group word.
 // The side distances of the cell mask cm and the next position; bias: what is added to the least
@@ -456,11 +464,12 @@ __device__ __forceinline__ i32x4 buffer_rsrc(const void* base, uint32_t stride, 
 // The sector record, loaded by the lanes that have entered another sector (lanes: what to save
 // exec in).
 #define VRT_STEP_RECORD(lanes)                                 \
-    "v_bfe_u32 %[t0], %[g0], 5, 15\n\t"                        \
-    "v_bfe_u32 %[t1], %[g1], 5, 15\n\t"                        \
-    "v_bfe_u32 %[t2], %[g2], 5, 15\n\t"                        \
+    "v_lshrrev_b32 %[t0], 5, %[g0]\n\t"                        \
+    "v_lshrrev_b32 %[t1], 5, %[g1]\n\t"                        \
+    "v_lshrrev_b32 %[t2], 5, %[g2]\n\t"                        \
     "v_mad_u32_u24 %[t2], %[t2], %[sz], %[t0]\n\t"             \
     "v_mad_u32_u24 %[t1], %[t1], %[sy], %[t2]\n\t"             \
+    "v_add_u32 %[t1], %[t1], %[sk]\n\t"                        \
     "v_cmp_ne_u32 vcc, %[t1], %[si]\n\t"                       \
     "s_and_saveexec_b64 " lanes ", vcc\n\t"                    \
     "s_cbranch_execz vrt_kept%=\n\t"                           \
@@ -538,7 +547,7 @@ __device__ __forceinline__ i32x4 buffer_rsrc(const void* base, uint32_t stride, 
     [o0] "v"(O[0]), [o1] "v"(O[1]), [o2] "v"(O[2]), [d0] "v"(D[0]), [d1] "v"(D[1]), [d2] "v"(D[2]),             \
         [i0] "v"(I[0]), [i1] "v"(I[1]), [i2] "v"(I[2]), [ts0] "v"(T[0]), [ts1] "v"(T[1]), [ts2] "v"(T[2]),      \
         [m0] "v"(M[0]), [m1] "v"(M[1]), [m2] "v"(M[2]), [b0] "v"(B[0]), [b1] "v"(B[1]), [b2] "v"(B[2]),         \
-        [max] "s"(cap), [sz] "s"(w.step_z), [sy] "s"(w.step_y), [rsec] "s"(rsec), [rocc] "s"(rocc)
+        [max] "s"(cap), [sz] "s"(w.step_z), [sy] "s"(w.step_y), [sk] "v"(step_bias(w)), [rsec] "s"(rsec), [rocc] "s"(rocc)
 #define VRT_STEP_CLOBBERS "v48", "v49", "v50", "v51", "v52", "v53", "v54", "v55", "vcc", "scc"
 
 // The fast loop, for quick or guarded rays.
