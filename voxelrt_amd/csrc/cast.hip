@@ -95,13 +95,15 @@ constexpr uint32_t kGridThreads = 64;
 // waves for the tail: 0.118 against 0.139 ms for the 1920x1080 primary rays.  A random
 // block order (0.145 ms) loses the L2 reuse between neighbouring tiles; in a window of 512
 // blocks each XCD takes neighbours (xcd_window_block).
+// shift: log2 of the rays of a wave, 6 or 0 (few_rays).
 template <bool COUNT, bool GROUPS>
 __global__ __launch_bounds__(kGridThreads) void cast_grid_kernel(WorldView w, RaysIn r, HitsOut h, uint32_t max_iters,
-                                                                 vrt_cast_counters* ctr, uint32_t reverse) {
+                                                                 vrt_cast_counters* ctr, uint32_t reverse,
+                                                                 uint32_t shift) {
     uint32_t blk = xcd_window_block(blockIdx.x, gridDim.x);
     if (reverse) blk = gridDim.x - 1u - blk;
-    uint32_t i = blk * kGridThreads + threadIdx.x;
-    bool valid = i < ray_count(r);
+    uint32_t i = (blk << shift) + threadIdx.x;
+    bool valid = i < ray_count(r) && threadIdx.x >> shift == 0;
     RayState st;
     float t = 0.0f;
     int4 rec = make_int4(0, 0, 0, 0);
@@ -464,6 +466,12 @@ static bool cast_by_groups(const WorldView& w, uint32_t n) {
     return (uint64_t)w.step_n * 16 > ((uint64_t)4 << 20) && n >= (1u << 18);
 }
 
+// Whether each ray of a grid cast gets a wave to itself.  A few rays leave the chip idle, and take as
+// long as the longest, whose wave's steps are shorter when no other lane is in a brick: 300 rays in the
+// 1024^3 terrain 31.6 -> 22.6 us, 1237 13.9 -> 13.3, 2500 37.6 -> 32.7, 4000 in the 2048^3 spheres 45.5 ->
+// 36.8.  From 4 waves per SIMD on they share its issue: 10 000 rays 39.8 -> 41.2.
+static bool few_rays(uint32_t n) { return n <= 4096; }
+
 // Option checks that do not depend on the ray count, so a call is rejected or
 // accepted the same way whatever n is (n = 0 included).
 int check_cast_opts(const vrt_cast_opts& o) {
@@ -509,11 +517,12 @@ int launch_cast(const vrt_world* world, const RaysIn& r, const HitsOut& h, uint3
         return VRT_OK;
     }
     if (sched == VRT_SCHED_GRID) {
-        uint32_t blocks = (uint32_t)(((uint64_t)r.n + kGridThreads - 1) / kGridThreads);
+        const uint32_t shift = few_rays(r.n) ? 0u : 6u;
+        uint32_t blocks = (uint32_t)(((uint64_t)r.n + (1u << shift) - 1) >> shift);
         uint32_t rev = o.order == VRT_ORDER_REVERSE ? 1u : 0u;
         auto* grid = o.counters ? (groups ? cast_grid_kernel<true, true> : cast_grid_kernel<true, false>)
                                 : (groups ? cast_grid_kernel<false, true> : cast_grid_kernel<false, false>);
-        grid<<<blocks, kGridThreads, 0, s>>>(w, r, h, max_iters, o.counters, rev);
+        grid<<<blocks, kGridThreads, 0, s>>>(w, r, h, max_iters, o.counters, rev, shift);
         VRT_HIP(hipGetLastError());
         return VRT_OK;
     }
