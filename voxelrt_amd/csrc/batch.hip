@@ -162,13 +162,13 @@ __device__ __forceinline__ void trace_block(const WorldView& w, const BatchArgs&
                 ray_hit_record(w, st[k], v[k], slot[k], t, rec);
             else
                 ray_miss_record(st[k], t, rec);
-            a.h.t[lr[k].out] = t;
-            a.h.rec[lr[k].out] = rec;
+            store_past(a.h.t + lr[k].out, t);
+            store_past(a.h.rec + lr[k].out, rec);
             if (a.h.pos_x) {
                 bool hit = (rec.w & 0xFF) != 0;
-                a.h.pos_x[lr[k].out] = hit ? st[k].cur[0] : 0.0f;
-                a.h.pos_y[lr[k].out] = hit ? st[k].cur[1] : 0.0f;
-                a.h.pos_z[lr[k].out] = hit ? st[k].cur[2] : 0.0f;
+                store_past(a.h.pos_x + lr[k].out, hit ? st[k].cur[0] : 0.0f);
+                store_past(a.h.pos_y + lr[k].out, hit ? st[k].cur[1] : 0.0f);
+                store_past(a.h.pos_z + lr[k].out, hit ? st[k].cur[2] : 0.0f);
             }
             if constexpr (COUNT) {
                 c_rays++;

@@ -50,24 +50,24 @@ __device__ __forceinline__ void flush_counters(vrt_cast_counters* ctr, unsigned 
 }
 
 __device__ __forceinline__ void store_result(const HitsOut& h, uint32_t i, const RayState& r, float t, int4 rec) {
-    h.t[i] = t;
-    h.rec[i] = rec;
+    store_past(h.t + i, t);
+    store_past(h.rec + i, rec);
     const bool hit = (rec.w & 0xFF) != 0;
     if (h.pos_x) {
-        h.pos_x[i] = hit ? r.cur[0] : 0.0f;
-        h.pos_y[i] = hit ? r.cur[1] : 0.0f;
-        h.pos_z[i] = hit ? r.cur[2] : 0.0f;
+        store_past(h.pos_x + i, hit ? r.cur[0] : 0.0f);
+        store_past(h.pos_y + i, hit ? r.cur[1] : 0.0f);
+        store_past(h.pos_z + i, hit ? r.cur[2] : 0.0f);
     }
     if (h.uv_u) {
         // UV of CpuRenderer.cpp:217-220: fract(X ? pos.y : pos.x), fract(Z ? pos.y : pos.z), the
         // tie masks X and Z being the nonzero normal fields of the record
         bool X = ((uint32_t)rec.w >> 8) & 3u, Z = ((uint32_t)rec.w >> 12) & 3u;
         float a = X ? r.cur[1] : r.cur[0], b = Z ? r.cur[1] : r.cur[2];
-        h.uv_u[i] = hit ? a - floorf(a) : 0.0f;
-        h.uv_v[i] = hit ? b - floorf(b) : 0.0f;
+        store_past(h.uv_u + i, hit ? a - floorf(a) : 0.0f);
+        store_past(h.uv_v + i, hit ? b - floorf(b) : 0.0f);
     }
     // the palette entry's low 32 bits (GetVoxelMaterial, CpuRenderer.cpp:120-132)
-    if (h.material_data) h.material_data[i] = hit ? (uint32_t)h.palette[rec.w & 0xFF] : 0u;
+    if (h.material_data) store_past(h.material_data + i, hit ? (uint32_t)h.palette[rec.w & 0xFF] : 0u);
 }
 
 __device__ __forceinline__ void finish_record(const WorldView& w, const RayState& st, bool hit, const int32_t v[3],
@@ -156,7 +156,8 @@ __global__ __launch_bounds__(kGridThreads) void cast_pass1_kernel(WorldView w, R
     RayState st;
     bool hit = false, survivor = false;
     if (valid) {
-        ray_setup(st, r.ox[i], r.oy[i], r.oz[i], r.dx[i], r.dy[i], r.dz[i], r.W[0], r.W[1], r.W[2]);
+        ray_setup(st, load_past(r.ox + i), load_past(r.oy + i), load_past(r.oz + i), load_past(r.dx + i),
+                  load_past(r.dy + i), load_past(r.dz + i), r.W[0], r.W[1], r.W[2]);
         int32_t v[3];
         uint32_t slot = 0;
         hit = ray_trace_wave<GROUPS>(w, st, cap, v, slot);
@@ -238,7 +239,8 @@ __global__ __launch_bounds__(kGridThreads) void cast_pass2_kernel(WorldView w, R
             const float4 a = q.a[i];
             const float2 b = q.b[i];
             RayState st;
-            ray_setup(st, r.ox[i], r.oy[i], r.oz[i], r.dx[i], r.dy[i], r.dz[i], r.W[0], r.W[1], r.W[2]);
+            ray_setup(st, load_past(r.ox + i), load_past(r.oy + i), load_past(r.oz + i), load_past(r.dx + i),
+                      load_past(r.dy + i), load_past(r.dz + i), r.W[0], r.W[1], r.W[2]);
             st.cur[0] = a.x;
             st.cur[1] = a.y;
             st.cur[2] = a.z;

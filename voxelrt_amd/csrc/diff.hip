@@ -80,8 +80,8 @@ __global__ __launch_bounds__(64) void render_fwd_kernel(WorldView w, FwdViews vi
         image[(size_t)i * 3 + 0] = r;
         image[(size_t)i * 3 + 1] = g;
         image[(size_t)i * 3 + 2] = b;
-        saved_voxel[i] = gv;
-        saved_weight[i] = wgt;
+        store_past(saved_voxel + i, gv);
+        store_past(saved_weight + i, wgt);
     }
 }
 

@@ -24,13 +24,13 @@
 namespace vrt {
 
 __device__ __forceinline__ void store_hit(const HitsOut& h, uint32_t i, const float* cur, float t, int4 rec) {
-    h.t[i] = t;
-    h.rec[i] = rec;
+    store_past(h.t + i, t);
+    store_past(h.rec + i, rec);
     if (h.pos_x) {
         bool hit = (rec.w & 0xFF) != 0;
-        h.pos_x[i] = hit ? cur[0] : 0.0f;
-        h.pos_y[i] = hit ? cur[1] : 0.0f;
-        h.pos_z[i] = hit ? cur[2] : 0.0f;
+        store_past(h.pos_x + i, hit ? cur[0] : 0.0f);
+        store_past(h.pos_y + i, hit ? cur[1] : 0.0f);
+        store_past(h.pos_z + i, hit ? cur[2] : 0.0f);
     }
 }
 

@@ -143,9 +143,10 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(7))) void re
     uint32_t ncode = 0;
 #pragma unroll
     for (int k = 0; k < 3; k++) ncode |= (uint32_t)(int32_t)(N[k] + 1.0f) << (2 * k);
-    a.albedo_normal[i] = unorm8(albedo[0]) | unorm8(albedo[1]) << 8 | unorm8(albedo[2]) << 16 | ncode << 24;
-    *(float4*)(a.irradiance + (size_t)i * 4) = make_float4(irr[0], irr[1], irr[2], (float)iters);
-    a.depth[i] = dep;
+    store_past(a.albedo_normal + i,
+               unorm8(albedo[0]) | unorm8(albedo[1]) << 8 | unorm8(albedo[2]) << 16 | ncode << 24);
+    store_past((float4*)(a.irradiance + (size_t)i * 4), make_float4(irr[0], irr[1], irr[2], (float)iters));
+    store_past(a.depth + i, dep);
 }
 
 }  // namespace

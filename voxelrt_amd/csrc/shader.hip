@@ -23,12 +23,13 @@ __global__ __launch_bounds__(256) void shader_cast_kernel(ShaderView sv, RaysIn 
     const int32_t W[3] = {r.W[0], r.W[1], r.W[2]};
     ShaderHit sh;
     bool hit = shader_trace<COARSE, LUT>(sv, lut, o, d, W, cap, sh);
-    h.t[i] = sh.t;
-    h.rec[i] = make_int4(sh.v[0], sh.v[1], sh.v[2], (int)(sh.mat | sh.code << 8 | (sh.iters & 0xFFFFu) << 16));
+    store_past(h.t + i, sh.t);
+    store_past(h.rec + i,
+               make_int4(sh.v[0], sh.v[1], sh.v[2], (int)(sh.mat | sh.code << 8 | (sh.iters & 0xFFFFu) << 16)));
     if (h.pos_x) {
-        h.pos_x[i] = hit ? sh.cur[0] : 0.0f;
-        h.pos_y[i] = hit ? sh.cur[1] : 0.0f;
-        h.pos_z[i] = hit ? sh.cur[2] : 0.0f;
+        store_past(h.pos_x + i, hit ? sh.cur[0] : 0.0f);
+        store_past(h.pos_y + i, hit ? sh.cur[1] : 0.0f);
+        store_past(h.pos_z + i, hit ? sh.cur[2] : 0.0f);
     }
 }
 
