@@ -225,7 +225,8 @@ typedef enum vrt_cast_schedule {
     VRT_SCHED_COMPACT = 3      /* cap and compact: a grid pass stops every ray after pass_cap steps;
                                   the rays still running are packed 64 to a wave and resumed from
                                   their saved state by a second pass.  For incoherent ray sets, whose
-                                  lanes finish at very different steps.  The survivor state (24 bytes
+                                  lanes finish at very different steps; below 2^19 rays, with pass_cap
+                                  0, one pass is faster and made.  The survivor state (24 bytes
                                   per ray of capacity and a 64-bit ballot per 64 rays) belongs to the
                                   (device, stream) pair; the first call on a stream, and a call with
                                   more rays than any before on it, allocates it (with a stream

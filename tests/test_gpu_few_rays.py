@@ -29,3 +29,12 @@ def test_few_rays(vrt, cuda, world, n, order):
         b = world.cast(rays, with_pos=True, schedule=PERSISTENT, counters=cb, count=limit)
         assert torch.equal(a.rec[:m], b.rec[:m]) and torch.equal(a.t[:m], b.t[:m])
         assert torch.equal(a.pos[:, :m], b.pos[:, :m]) and torch.equal(ca, cb)
+
+
+@pytest.mark.parametrize("n", [1, 4097, (1 << 19) - 1, 1 << 19, (1 << 19) + 65])
+def test_compact_schedule_around_its_second_pass(vrt, cuda, world, n):
+    rays = vrt.RayBatch.from_numpy(*random_rays(n, 128, seed=n, inside=False))
+    want = world.cast(rays, with_pos=True, schedule=PERSISTENT)
+    for cap in (0, 3, 32):
+        got = world.cast(rays, with_pos=True, schedule=3, pass_cap=cap)
+        assert torch.equal(got.rec, want.rec) and torch.equal(got.t, want.t) and torch.equal(got.pos, want.pos), cap

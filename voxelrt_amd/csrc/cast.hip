@@ -458,6 +458,11 @@ static int survivor_state(int dev, hipStream_t s, uint32_t n, SurvivorState* q) 
 // 24, against 0.341 ms for the grid); 64 is best in the 587-sphere world (0.432 against
 // 0.448 ms).
 constexpr uint32_t kDefaultPassCap = 32;
+// Rays from which the compact schedule makes two passes when the caller leaves the cap to it; fewer
+// leave SIMDs idle in the second.  Rays without order, one pass against two: 100 k in the 2048^3 spheres
+// 85 and 92 us, in the 1024^3 terrain 61 and 70, in 512^3 45 and 55; 400 k 112 and 120, 84 and 92, 56
+// and 65; 800 k 190 and 169, 137 and 138, 78 and 89; 2 M 412 and 350, 284 and 271, 155 and 160.
+constexpr uint32_t kCompactRays = 1u << 19;
 
 // Whether a cast reads the group table first (ray_trace_fast): where the step table no longer fits an
 // XCD's 4 MiB L2, and there are enough rays to be bound by the requests to it.  2 M rays without
@@ -497,11 +502,14 @@ int launch_cast(const vrt_world* world, const RaysIn& r, const HitsOut& h, uint3
     // a first pass as long as the cast is the whole cast
     if (sched == VRT_SCHED_COMPACT && cap >= max_iters) sched = VRT_SCHED_GRID;
     const bool groups = cast_by_groups(w, r.n);
+    SurvivorState q;
     if (sched == VRT_SCHED_COMPACT) {
-        SurvivorState q;
-        int rc;
-        rc = survivor_state(world->device, s, r.n, &q);
+        int rc = survivor_state(world->device, s, r.n, &q);
         if (rc != VRT_OK) return rc;
+        // one pass, with the state as for two: a later capture on the stream may need it
+        if (!o.pass_cap && r.n < kCompactRays) sched = VRT_SCHED_GRID;
+    }
+    if (sched == VRT_SCHED_COMPACT) {
         const uint32_t blocks = (uint32_t)(((uint64_t)r.n + kGridThreads - 1) / kGridThreads);
         const uint32_t rev = o.order == VRT_ORDER_REVERSE ? 1u : 0u;
         // pass 2: 64 rounds per group of 64 ray blocks (a round past a group's survivors exits)
