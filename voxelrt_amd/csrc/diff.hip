@@ -292,11 +292,13 @@ __global__ __launch_bounds__(256) void bwd_place_kernel(uint32_t n, const float*
                                                         float4* __restrict__ list) {
     const uint32_t i = blockIdx.x * 256 + threadIdx.x;
     if (i >= n) return;
-    const uint32_t r = rank[i], gv = saved_voxel[i];
+    const uint32_t r = rank[i];
+    if (r == 0xFFFFFFFFu) return;
+    const uint32_t gv = saved_voxel[i];
     const float w = saved_weight[i];
     const float x = grad_image[(size_t)i * 3 + 0] * w, y = grad_image[(size_t)i * 3 + 1] * w,
                 z = grad_image[(size_t)i * 3 + 2] * w;
-    if (r != 0xFFFFFFFFu) list[offsets[gv >> 9] + r] = make_float4(x, y, z, __uint_as_float(gv & 511u));
+    list[offsets[gv >> 9] + r] = make_float4(x, y, z, __uint_as_float(gv & 511u));
 }
 
 // Pass 4: one workgroup per touched slot, striding over them (their number is on the device).  The
