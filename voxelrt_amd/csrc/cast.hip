@@ -465,12 +465,16 @@ constexpr uint32_t kDefaultPassCap = 32;
 constexpr uint32_t kCompactRays = 1u << 19;
 
 // Whether a cast reads the group table first (ray_trace_fast): where the step table no longer fits an
-// XCD's 4 MiB L2, and there are enough rays to be bound by the requests to it.  2 M rays without
-// order in the 2048^3 world of 587 spheres (a table of 4.8 MB): compact 497 -> 376 us, grid
-// 484 -> 421; its 1920x1080 primary rays 63.5 -> 64.4, 300 k rays 109 -> 104, 100 k 96 -> 105.  In
-// the 1024^3 terrain (0.7 MB) 2 M such rays gain 7% and 0.25 M lose 18%; in 512^3 both lose 14%.
-static bool cast_by_groups(const WorldView& w, uint32_t n) {
-    return (uint64_t)w.step_n * 16 > ((uint64_t)4 << 20) && n >= (1u << 18);
+// XCD's 4 MiB L2, there are enough rays to be bound by the requests to it, and enough sectors are
+// empty for the group's word to spare them.  2 M rays without order in the 2048^3 worlds of 587 to
+// 20 000 spheres (a table of 4.8 MB), by the share of sectors with a brick, with groups and without:
+// grid 0.06 381 and 442 us, 0.14 419 and 430, 0.27 440 and 417, 0.87 368 and 318; compact 0.06 341 and
+// 464, 0.27 379 and 421, 0.47 358 and 374, 0.65 359 and 339, 0.87 326 and 295.  At 0.06 the 1920x1080
+// primary rays 63.5 -> 64.4, 300 k rays 109 -> 104, 100 k 96 -> 105.  In the 1024^3 terrain (0.7 MB) 2 M
+// such rays gain 7% and 0.25 M lose 18%; in 512^3 both lose 14%.
+static bool cast_by_groups(const vrt_world* world, const WorldView& w, uint32_t n, bool compact) {
+    return (uint64_t)w.step_n * 16 > ((uint64_t)4 << 20) && n >= (1u << 18) &&
+           world->full_sectors <= world->nsec / (compact ? 2 : 5);
 }
 
 // Whether each ray of a grid cast gets a wave to itself.  A few rays leave the chip idle, and take as
@@ -501,7 +505,6 @@ int launch_cast(const vrt_world* world, const RaysIn& r, const HitsOut& h, uint3
     const uint32_t cap = o.pass_cap ? o.pass_cap : kDefaultPassCap;
     // a first pass as long as the cast is the whole cast
     if (sched == VRT_SCHED_COMPACT && cap >= max_iters) sched = VRT_SCHED_GRID;
-    const bool groups = cast_by_groups(w, r.n);
     SurvivorState q;
     if (sched == VRT_SCHED_COMPACT) {
         int rc = survivor_state(world->device, s, r.n, &q);
@@ -509,6 +512,7 @@ int launch_cast(const vrt_world* world, const RaysIn& r, const HitsOut& h, uint3
         // one pass, with the state as for two: a later capture on the stream may need it
         if (!o.pass_cap && r.n < kCompactRays) sched = VRT_SCHED_GRID;
     }
+    const bool groups = cast_by_groups(world, w, r.n, sched == VRT_SCHED_COMPACT);
     if (sched == VRT_SCHED_COMPACT) {
         const uint32_t blocks = (uint32_t)(((uint64_t)r.n + kGridThreads - 1) / kGridThreads);
         const uint32_t rev = o.order == VRT_ORDER_REVERSE ? 1u : 0u;

@@ -181,6 +181,7 @@ struct vrt_world {
     std::vector<uint32_t> h_base;
     vrt::SlotArena arena;
     uint32_t num_bricks = 0;
+    uint32_t full_sectors = 0;        // sectors that hold a brick
     // shader method: sector-of-sectors masks and the ray-cell table
     uint32_t gshift_xz = 0, gshift_y = 0;
     std::vector<uint64_t> h_groups;

@@ -614,6 +614,7 @@ static int world_sync(vrt_world* w, uint32_t nsec, const uint32_t* sector_idx, c
         uint32_t idx = sector_idx[i];
         w->num_bricks -= (uint32_t)std::popcount(w->h_mask[idx]);
         w->num_bricks += (uint32_t)std::popcount(alloc_mask[i]);
+        w->full_sectors += (uint32_t)(alloc_mask[i] != 0) - (uint32_t)(w->h_mask[idx] != 0);
         w->h_mask[idx] = alloc_mask[i];
         w->h_base[idx] = new_base[i];
     }
