@@ -556,9 +556,9 @@ int vrt_render_bwd(const vrt_world* world, uint32_t npixels, const float* grad_i
 /*
  * The same gradient, every one of the nvox * 3 entries written (no zeroing beforehand):
  * grad_albedo[v][c] = sum over pixels hitting v of grad_image[p][c] * saved_weight[p], 0 for
- * voxels no pixel hit.  Hit pixels are bucketed by brick slot (a counting sort), then each
- * slot's contributions are summed in LDS and its 512 rows written once; no global float
- * atomics.  nvox >= vrt_world_info.slot_high_water * 512 (the albedo's length); grad_albedo
+ * voxels no pixel hit.  Zeros are written first; hit pixels are bucketed by brick slot (a
+ * counting sort), then each hit slot's contributions are summed in LDS, in 64 bits, and its 512
+ * rows written; no global float atomics.  nvox >= vrt_world_info.slot_high_water * 512 (the albedo's length); grad_albedo
  * 16-byte aligned; workspace (256-byte aligned) of vrt_render_bwd_workspace_bytes(npixels,
  * nvox) bytes.  The summation order within a voxel is not fixed (LDS atomics).
  */
