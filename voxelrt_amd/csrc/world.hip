@@ -324,7 +324,8 @@ static int ensure_staging(vrt_world* w) {
     uint8_t* h = nullptr;
     uint8_t* d = nullptr;
     hipEvent_t ev[2] = {nullptr, nullptr};
-    hipError_t e = hipHostMalloc((void**)&h, 2 * kSyncHalf, hipHostMallocDefault);
+    // coherent whatever the environment's default: kernels read it (kSyncDirect)
+    hipError_t e = hipHostMalloc((void**)&h, 2 * kSyncHalf, hipHostMallocCoherent);
     if (e == hipSuccess) e = hipMalloc(&d, 2 * kSyncHalf);
     if (e == hipSuccess) e = hipEventCreateWithFlags(&ev[0], hipEventDisableTiming);
     if (e == hipSuccess) e = hipEventCreateWithFlags(&ev[1], hipEventDisableTiming);
@@ -685,7 +686,7 @@ int vrt_world_create(const vrt_world_desc* desc, void* stream, vrt_world** out) 
         const size_t o_groups = part(w->h_groups.size() * 8), o_sgroups = part((size_t)w->group_n() * 8);
         const size_t o_palette = part(256 * 8), o_lut = part(512 * 8);
         check(hipMalloc(&w->d_tables, bytes), "hipMalloc(world tables)");
-        check(hipHostMalloc(&w->h_pick, kPickBytes, hipHostMallocDefault), "hipHostMalloc(picking result)");
+        check(hipHostMalloc(&w->h_pick, kPickBytes, hipHostMallocCoherent), "hipHostMalloc(picking result)");
         if (rc == VRT_OK) {
             std::memset(w->h_pick, 0, kPickBytes);
             w->d_sec = (uint4*)(w->d_tables + o_sec);
