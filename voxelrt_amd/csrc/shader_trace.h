@@ -210,7 +210,11 @@ __device__ __forceinline__ uint32_t fill_lut(const ShaderView& sv, uint4* lut) {
 // shader_loop for quick rays (ray_is_quick of the start org, d and inv): the cast's fast loop
 // (traverse.h) with this method's bias, its level above an empty sector (step records' bits 8..9) and
 // rayCastCoarse's stop in a non-empty cell from step 31 on.  The largest cell, 128 voxels, lies inside
-// the tables, so positions stay within their border as there.  A step at the sector level takes 37 vector
+// the tables.  Positions stay within their border as there where the distances run from a point of the
+// world (rayCastCoarse: from the clipped start).  rayCast's run from the origin itself, so that t covers
+// the way to the world and both its rounding and the bias of 5 ulps grow with it: past a cell's far plane
+// by up to 2^-23 |o| and 5 2^-23 |o| voxels of each axis.  With |o| below 2^24 on every axis that is 12 of
+// the border's 32; rays from further away take shader_loop (ray_starts_near).  A step at the sector level takes 37 vector
 // instructions (shader_loop's about 70, with no record kept between steps): 2.07 M camera rays over
 // the 1024^3 terrain 167 -> 96 us (rayCast), 80 -> 45 us (rayCastCoarse).  slot: the hit voxel's
 // brick.  With the ray-cell table (lut: fill_lut's result plus the ray's octant * 512) a step ands
@@ -298,6 +302,12 @@ __device__ __forceinline__ bool shader_loop_fast(const ShaderView& sv, uint32_t 
     return hit;
 }
 
+// Whether rayCast's distances, taken from o, keep a ray's positions within the border (shader_loop_fast).
+// From 2^26 on they do not: nearly parallel rays then miss the border's records.
+__device__ __forceinline__ bool ray_starts_near(const float o[3]) {
+    return fmaxf(fmaxf(fabsf(o[0]), fabsf(o[1])), fabsf(o[2])) < 16777216.0f;
+}
+
 // rayCast (COARSE = false, :162-204) or rayCastCoarse (COARSE = true, :206-243).  lut: fill_lut's result.
 template <bool COARSE, bool LUT>
 __device__ __forceinline__ bool shader_trace(const ShaderView& sv, uint32_t lut, const float o[3], const float d[3],
@@ -322,7 +332,7 @@ __device__ __forceinline__ bool shader_trace(const ShaderView& sv, uint32_t lut,
 #pragma unroll
     for (int a = 0; a < 3; a++) inv[a] = reciprocal_in_range(d[a]);
     begin();
-    if (origin_is_guarded(W) && __all(ray_is_quick(org, d, inv))) {
+    if (origin_is_guarded(W) && __all(ray_is_quick(org, d, inv) && (COARSE || ray_starts_near(org)))) {
         hit = shader_loop_fast<COARSE, LUT>(sv, lut + oct * 512u, d, org, inv, ts, W, dm, cap, v, side, cur, tmin, it,
                                             slot);
     } else {
