@@ -1,4 +1,4 @@
-"""Build script for libvoxelrt_hip.so (gfx950) and the oracle library.
+"""Build script for libvoxelrt_hip.so (gfx950), the oracle library and the tests' own kernels.
 
 Run ``python -m voxelrt_amd.build`` (or ``__graft_entry__.build()``).  Every
 call recompiles: sources are few and hipcc takes seconds per file.
@@ -97,6 +97,25 @@ def build_torch_extension(verbose: bool = True) -> Path:
     return TORCH_EXT
 
 
+CHECKS = ROOT / "tests" / "hip" / "libdevice_checks.so"
+
+
+def build_checks(verbose: bool = True) -> Path:
+    """What tests/test_gpu_device_facts.py calls beside the ABI: test infrastructure, loaded by that test alone
+    (linked against libvoxelrt_hip.so, found through $ORIGIN)."""
+    src = CHECKS.parent / "device_checks.hip"
+    tmp = CHECKS.with_suffix(".so.tmp")
+    cmd = [HIPCC, *HIP_FLAGS, "-shared", str(src), "-o", str(tmp), f"-L{PKG}", "-lvoxelrt_hip",
+           "-Wl,-rpath,$ORIGIN/../../voxelrt_amd"]
+    res = subprocess.run(cmd, capture_output=True, text=True)
+    if res.returncode != 0:
+        raise RuntimeError(f"hipcc failed for {src}:\n{' '.join(cmd)}\n{res.stdout}\n{res.stderr}")
+    os.replace(tmp, CHECKS)
+    if verbose:
+        print(f"built {CHECKS.relative_to(ROOT)}", flush=True)
+    return CHECKS
+
+
 def build_oracle(verbose: bool = True) -> Path:
     """The oracle is test infrastructure (the checker and CPU baseline)."""
     make = shutil.which("make")
@@ -113,6 +132,7 @@ def build_oracle(verbose: bool = True) -> Path:
 def build_all(verbose: bool = True) -> None:
     build_library(verbose)
     build_torch_extension(verbose)
+    build_checks(verbose)
     build_oracle(verbose)
 
 

@@ -332,7 +332,8 @@ __device__ __forceinline__ bool shader_trace(const ShaderView& sv, uint32_t lut,
 #pragma unroll
     for (int a = 0; a < 3; a++) inv[a] = reciprocal_in_range(d[a]);
     begin();
-    if (origin_is_guarded(W) && __all(ray_is_quick(org, d, inv) && (COARSE || ray_starts_near(org)))) {
+    if (origin_is_guarded(W) && masks_in_reach(w) &&
+        __all(ray_is_quick(org, d, inv) && (COARSE || ray_starts_near(org)))) {
         hit = shader_loop_fast<COARSE, LUT>(sv, lut + oct * 512u, d, org, inv, ts, W, dm, cap, v, side, cur, tmin, it,
                                             slot);
     } else {

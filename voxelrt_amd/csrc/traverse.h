@@ -377,6 +377,11 @@ __device__ __forceinline__ bool origin_is_guarded(const int32_t W[3]) {
     return ok;
 }
 
+// Whether a structured load reaches every mask.  This part cuts its index times its stride to 32 bits
+// (index 2^29 of a table of 8-byte records reads record 0), and the base is a slot early (ray_trace_fast).
+// Worlds that hold memory for more bricks than 2^26 - 1 take ray_advance's step, with 64-bit addresses.
+__device__ __forceinline__ bool masks_in_reach(const WorldView& w) { return w.occ_n <= (1u << 29) - 8u; }
+
 // cur + bias per axis, rounded down.
 __device__ __forceinline__ void biased_floor(const float cur[3], const float bias[3], uint32_t g[3]) {
     asm("s_setreg_imm32_b32 hwreg(HW_REG_MODE, 0, 2), 2\n\t"
@@ -637,7 +642,7 @@ __device__ __forceinline__ bool ray_trace_steps(const WorldView& w, RayState& r,
 template <bool GROUPS = false>
 __device__ __forceinline__ bool ray_trace_wave(const WorldView& w, RayState& r, uint32_t max_iters, int32_t v[3],
                                                uint32_t& slot, uint32_t first = 0) {
-    const bool near = origin_is_guarded(r.W);  // uniform
+    const bool near = origin_is_guarded(r.W) && masks_in_reach(w);  // uniform
     if (!(near && __all(ray_is_quick(r.o, r.d, r.inv)))) {
         ray_exact_inverse(r);
         const bool tame = __all(ray_is_tame(r));
