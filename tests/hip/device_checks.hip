@@ -1,6 +1,6 @@
-// device_checks.hip - what tests/test_gpu_device_facts.py calls beside the ABI: kernels for facts about this
-// part that the traversal's loops rest on, through the functions that the loops use (traverse.h), and a
-// world's slot arena.
+// device_checks.hip - what tests/test_gpu_device_facts.py and test_bwd_large.py call beside the ABI: kernels
+// for facts about this part that the traversal's loops rest on, through the functions that the loops use
+// (traverse.h), a world's slot arena, and the split of large launches.
 #include <hip/hip_runtime.h>
 
 #include "traverse.h"
@@ -52,6 +52,14 @@ int check_structured_loads(const void* table, uint32_t stride, uint32_t records,
 int check_take_slots(vrt_world* world, uint32_t n) {
     uint32_t base = 0;
     return world->arena.realloc(base, 0, n) && base == 0 ? 0 : 1;
+}
+
+// Blocks of each launch of a kernel of `blocks` blocks in all; their number.
+uint32_t check_launches(uint64_t blocks, uint32_t threads, uint32_t* each, uint32_t max) {
+    uint32_t n = 0;
+    for (uint64_t first = 0; first < blocks && n < max; first += each[n++])
+        each[n] = vrt::launch_blocks(blocks - first, threads);
+    return n;
 }
 
 }  // extern "C"

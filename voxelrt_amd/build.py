@@ -101,8 +101,8 @@ CHECKS = ROOT / "tests" / "hip" / "libdevice_checks.so"
 
 
 def build_checks(verbose: bool = True) -> Path:
-    """What tests/test_gpu_device_facts.py calls beside the ABI: test infrastructure, loaded by that test alone
-    (linked against libvoxelrt_hip.so, found through $ORIGIN)."""
+    """What some tests call beside the ABI (test infrastructure, loaded by no one else): linked against
+    libvoxelrt_hip.so, found through $ORIGIN."""
     src = CHECKS.parent / "device_checks.hip"
     tmp = CHECKS.with_suffix(".so.tmp")
     cmd = [HIPCC, *HIP_FLAGS, "-shared", str(src), "-o", str(tmp), f"-L{PKG}", "-lvoxelrt_hip",

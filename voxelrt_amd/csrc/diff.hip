@@ -154,10 +154,11 @@ constexpr uint32_t kScanBlock = 1024;   // slots per block of the allocation
 
 // Zeros in `vecs` float4s from `out` and the `tail` floats after them, and in `n` words of p.  A float4
 // per thread, so that neighbouring blocks fill neighbouring 4 KB: 6.9 TB/s (blocks of 16 and 64 KB
-// reach 6.1 and 5.1, grids that stride over the gradient 4.4-6.1).
+// reach 6.1 and 5.1, grids that stride over the gradient 4.4-6.1).  first: the launch's first block, as
+// gradients past 68 GB need more lanes than a launch has.
 __global__ __launch_bounds__(256) void bwd_fill_kernel(float4* __restrict__ out, uint64_t vecs, uint32_t tail,
-                                                       uint32_t* __restrict__ p, uint32_t n) {
-    const uint64_t v = (uint64_t)blockIdx.x * 256 + threadIdx.x;
+                                                       uint32_t* __restrict__ p, uint32_t n, uint64_t first) {
+    const uint64_t v = (first + blockIdx.x) * 256 + threadIdx.x;
     if (v < vecs)
         out[v] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
     else if (v - vecs < tail)
@@ -508,19 +509,28 @@ int vrt_render_bwd_bricks(const vrt_world* world, uint32_t npixels, const float*
         // kernels, not memsets (graph-safe); the counts and cursors are cleared with the gradient
         const uint64_t vecs = nvox * 3 / 4;
         const uint32_t tail = (uint32_t)(nvox * 3 % 4), words = npixels ? ns + kCursorWords : 0u;
-        bwd_fill_kernel<<<(uint32_t)((vecs + tail + words + 255) / 256), 256, 0, s>>>((float4*)grad_albedo, vecs, tail,
-                                                                                     ws.cursor, words);
+        const uint64_t fill = (vecs + tail + words + 255) / 256;
+        for (uint64_t first = 0; first < fill;) {
+            const uint32_t blocks = launch_blocks(fill - first, 256);
+            bwd_fill_kernel<<<blocks, 256, 0, s>>>((float4*)grad_albedo, vecs, tail, ws.cursor, words, first);
+            // every pass indexes by what the passes before it wrote: none after one that failed
+            VRT_HIP(hipGetLastError());
+            first += blocks;
+        }
         if (npixels) {
             bwd_count_kernel<<<(npixels + kCountThreads - 1) / kCountThreads, kCountThreads, 0, s>>>(
                 npixels, saved_voxel, saved_weight, ws.counts, ws.rank);
+            VRT_HIP(hipGetLastError());
             bwd_alloc_kernel<<<nblk, 256, 0, s>>>(ns, ws.counts, ws.cursor, ws.offsets, ws.touched);
+            VRT_HIP(hipGetLastError());
             bwd_place_kernel<<<(npixels + 255) / 256, 256, 0, s>>>(npixels, grad_image, saved_voxel, saved_weight, ws.rank,
                                                                    ws.offsets, ws.list);
+            VRT_HIP(hipGetLastError());
             const uint32_t blocks = std::min({ns, npixels, kReduceBlocks});
             bwd_reduce_kernel<<<(blocks + 7) / 8 * 8, kReduceThreads, 0, s>>>(nvox, ws.cursor, ws.touched, ws.list,
                                                                              grad_albedo);
+            VRT_HIP(hipGetLastError());
         }
-        VRT_HIP(hipGetLastError());
         return VRT_OK;
     });
 }

@@ -3,6 +3,7 @@
 
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <cstdint>
 #include <map>
 #include <mutex>
@@ -266,6 +267,11 @@ namespace vrt {
 constexpr size_t kPickBytes = 64;
 // Bytes of one sync staging half (host pinned and device).
 constexpr size_t kSyncHalf = (size_t)8 << 20;
+
+// Blocks of the next launch of a kernel that needs `left` more: a launch has fewer than 2^32 lanes.
+inline uint32_t launch_blocks(uint64_t left, uint32_t threads) {
+    return (uint32_t)std::min<uint64_t>(left, 0xFFFFFFFFu / threads);
+}
 
 // VRT_OK, or VRT_ERR_STATE (with the message) when a failed sync left the world unusable.
 int check_world(const vrt_world* w, const char* entry);
