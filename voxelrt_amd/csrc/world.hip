@@ -704,6 +704,8 @@ int vrt_world_create(const vrt_world_desc* desc, void* stream, vrt_world** out) 
             world_init_kernel<<<(n + 255) / 256, 256, 0, s>>>(t);
             check(hipGetLastError(), "world_init_kernel");
             check(hipMemcpyAsync(w->d_lut, lut.data(), 512 * 8, hipMemcpyHostToDevice, s), "hipMemcpyAsync(ray-cell table)");
+            // the tables are whole when the call returns: a program may go on on another stream
+            check(hipStreamSynchronize(s), "hipStreamSynchronize(world tables)");
         }
         if (rc == VRT_OK && desc->initial_slots) rc = grow_slots(w, std::min(desc->initial_slots, w->arena.capacity()), s);
         if (rc == VRT_OK) check(hipStreamSynchronize(s), "hipStreamSynchronize");
