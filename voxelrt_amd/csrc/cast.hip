@@ -464,16 +464,23 @@ constexpr uint32_t kDefaultPassCap = 32;
 // and 65; 800 k 190 and 169, 137 and 138, 78 and 89; 2 M 412 and 350, 284 and 271, 155 and 160.
 constexpr uint32_t kCompactRays = 1u << 19;
 
-// Whether a cast reads the group table first (ray_trace_fast): where the step table no longer fits an
+// Whether a cast reads the group table first (ray_trace_fast): where the world's own step records fill an
 // XCD's 4 MiB L2, there are enough rays to be bound by the requests to it, and enough sectors are
 // empty for the group's word to spare them.  2 M rays without order in the 2048^3 worlds of 587 to
-// 20 000 spheres (a table of 4.8 MB), by the share of sectors with a brick, with groups and without:
+// 20 000 spheres (records of 4 MiB), by the share of sectors with a brick, with groups and without:
 // grid 0.06 381 and 442 us, 0.14 419 and 430, 0.27 440 and 417, 0.87 368 and 318; compact 0.06 341 and
 // 464, 0.27 379 and 421, 0.47 358 and 374, 0.65 359 and 339, 0.87 326 and 295.  At 0.06 the 1920x1080
-// primary rays 63.5 -> 64.4, 300 k rays 109 -> 104, 100 k 96 -> 105.  In the 1024^3 terrain (0.7 MB) 2 M
+// primary rays 63.5 -> 64.4, 300 k rays 109 -> 104, 100 k 96 -> 105.  In the 1024^3 terrain (0.5 MB) 2 M
 // such rays gain 7% and 0.25 M lose 18%; in 512^3 both lose 14%.
-static bool cast_by_groups(const vrt_world* world, const WorldView& w, uint32_t n, bool compact) {
-    return (uint64_t)w.step_n * 16 > ((uint64_t)4 << 20) && n >= (1u << 18) &&
+// Flat worlds, a word of whose groups covers few sectors and whose rays leave after few steps, at shares of
+// 0.05 and 0.15, with groups and without.  Records of 1 MiB (8192x32x8192): grid 185 and 172, 211 and 179,
+// compact 143 and 141, 161 and 141; of 2 MiB (8192x64x8192): 206 and 193, 242 and 207, 168 and 169, 190 and
+// 168.  Of 4 MiB one and four sectors high: grid 214 and 200, 249 and 207; 237 and 241, 281 and 248;
+// compact 167 and 175, 184 and 179; 196 and 217, 224 and 221.  Of 8 MiB two high: grid 234 and 233, 271 and
+// 242, compact 185 and 225, 210 and 228; of 16 MiB four high: grid 263 and 306, 300 and 306.  So the grid
+// needs whole groups.
+static bool cast_by_groups(const vrt_world* world, uint32_t n, bool compact) {
+    return world->nsec >= (1u << 18) && n >= (1u << 18) && (compact || world->shift_y >= 2) &&
            world->full_sectors <= world->nsec / (compact ? 2 : 5);
 }
 
@@ -512,7 +519,7 @@ int launch_cast(const vrt_world* world, const RaysIn& r, const HitsOut& h, uint3
         // one pass, with the state as for two: a later capture on the stream may need it
         if (!o.pass_cap && r.n < kCompactRays) sched = VRT_SCHED_GRID;
     }
-    const bool groups = cast_by_groups(world, w, r.n, sched == VRT_SCHED_COMPACT);
+    const bool groups = cast_by_groups(world, r.n, sched == VRT_SCHED_COMPACT);
     if (sched == VRT_SCHED_COMPACT) {
         const uint32_t blocks = (uint32_t)(((uint64_t)r.n + kGridThreads - 1) / kGridThreads);
         const uint32_t rev = o.order == VRT_ORDER_REVERSE ? 1u : 0u;
