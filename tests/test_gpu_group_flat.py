@@ -38,3 +38,14 @@ def test_flat_worlds(vrt, cuda, log2_y, share):
             got = world.cast(rays, schedule=schedule, pass_cap=cap, with_pos=True)
             assert torch.equal(got.rec, ref.rec) and torch.equal(got.t, ref.t), (W, schedule, cap)
             assert torch.equal(got.pos, ref.pos), (W, schedule, cap)
+
+
+@pytest.mark.parametrize("log2_xz,log2_y", [(13, 5), (12, 7), (5, 14), (8, 8)])
+def test_tables_hold_the_world_and_its_border(vrt, cuda, log2_xz, log2_y):
+    """Device memory of a world without bricks: the sector records, and two tables of 16-byte records with one
+    sector of border around at least 4x4x4 sectors.  The rest (group words, palette, ray-cell table) is small."""
+    nxz, ny = 1 << (log2_xz - 5), 1 << (log2_y - 5)
+    tables = 16 * nxz * nxz * ny + 2 * 16 * (max(nxz, 4) + 2) ** 2 * (max(ny, 4) + 2)
+    groups = 8 * (max(nxz // 4, 1) + 2) ** 2 * (max(ny // 4, 1) + 2) * 2
+    info = vrt.World(log2_xz, log2_y).info()
+    assert tables <= info.device_bytes <= tables + groups + 8192

@@ -403,12 +403,13 @@ __device__ __forceinline__ i32x4 buffer_rsrc(const void* base, uint32_t stride, 
     return r;
 }
 
-// What the record's index is too large by with the coordinates' exponent bits left in: 2^23's bits
-// >> 5, of which the products take the low 24.  Negated.  (Taking them out of each coordinate is
-// three bitfield extracts of 4 cycles for three shifts of 2 and an addition: 0.6% on the frames.)
+// What the record's index is too large by with the border's first sector and the coordinates' exponent
+// bits left in: 2^23's bits >> 5, of which the products take the low 24.  Negated.  (Taking the bits out of
+// each coordinate is three bitfield extracts of 4 cycles for three shifts of 2 and an addition: 0.6% on
+// the frames.)
 __device__ __forceinline__ uint32_t step_bias(const WorldView& w) {
     constexpr uint32_t e = 0x4B000000u >> 5, e24 = e & 0xFFFFFFu;
-    return 0u - (e + e24 * w.step_z + e24 * w.step_y);
+    return 0u - (e + kStepFirst + (e24 + kStepFirst) * (w.step_z + w.step_y));
 }
 
 // The parts of the fast loop (operands: ray_trace_fast).  Fixed registers: v[48:51] the kept

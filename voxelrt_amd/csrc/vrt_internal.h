@@ -90,14 +90,15 @@ __host__ __device__ inline uint4 sector_record(uint64_t mask, uint32_t base) {
 // step that leaves the world lands in the border and needs no bounds test.  Their indices come
 // from padded coordinates, the voxel's plus kStepPad (one group of 4x4x4 sectors) on each axis.
 constexpr int32_t kStepPad = 128;
+constexpr uint32_t kStepFirst = 3;
 // The group table: per group of 4x4x4 sectors a u64, bit x | z << 2 | y << 4 set when that sector
 // has a brick or lies outside the world.  Group (X, Y, Z) of the padded coordinates (>> 7) is word
 // X + Z * group_z + Y * group_y.
 // The step table: per sector a 16-byte record, and border records around them: one sector before the
 // world, and after it up to one past the world's last sector or the group of 4, whichever is
 // further (the shader method's cells are up to a group wide).
-// Sector (X, Y, Z) of the padded coordinates (>> 5; the world's first is 4, the border's 3) is
-// record X + Z * step_z + Y * step_y; the records before the border's first are never read.
+// Sector (X, Y, Z) of the padded coordinates (>> 5; the world's first is 4, the border's kStepFirst) is
+// record X - kStepFirst + (Z - kStepFirst) * step_z + (Y - kStepFirst) * step_y.
 //   x, y  allocation mask; all ones in the border (the step's brick test then succeeds)
 //   z     base slot; all ones in the border (base slots are below 2^28)
 //   w     per 2x2x2 group of bricks (gx, gz, gy = bit 4 of x, z, y) the cell mask of a step that
@@ -217,8 +218,7 @@ struct vrt_world {
     // at least 4 sectors a side and the border
     uint32_t step_z() const { return std::max(4u, 1u << shift_xz) + 2u; }
     uint32_t step_y() const { return step_z() * step_z(); }
-    uint32_t step_first() const { return 3u + 3u * step_z() + 3u * step_y(); }
-    uint32_t step_n() const { return step_first() + step_y() * (std::max(4u, 1u << shift_y) + 2u); }
+    uint32_t step_n() const { return step_y() * (std::max(4u, 1u << shift_y) + 2u); }
     uint32_t group_z() const { return (1u << gshift_xz) + 2u; }
     uint32_t group_y() const { return group_z() * group_z(); }
     uint32_t group_n() const { return group_y() * ((1u << gshift_y) + 2u); }

@@ -181,15 +181,14 @@ __global__ __launch_bounds__(256) void sync_place_kernel(uint8_t* __restrict__ v
 struct WorldTables {
     uint4 *sec, *steps, *masks;
     uint64_t *groups, *sgroups, *palette;
-    uint32_t nsec, step_z, step_y, step_first, step_n, nxz, ny, ngroups, group_z, group_y, group_n;
+    uint32_t nsec, step_z, step_y, step_n, nxz, ny, ngroups, group_z, group_y, group_n;
     uint64_t outside;
 };
 __global__ __launch_bounds__(256) void world_init_kernel(WorldTables t) {
     const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i < t.nsec) t.sec[i] = sector_record(0, 0);
     if (i < t.step_n) {
-        const uint32_t k = i < t.step_first ? 0u : i - t.step_first;
-        const uint32_t y = k / t.step_y, z = k % t.step_y / t.step_z, x = k % t.step_z;
+        const uint32_t y = i / t.step_y, z = i % t.step_y / t.step_z, x = i % t.step_z;
         const bool border = x == 0 || x > t.nxz || z == 0 || z > t.nxz || y == 0 || y > t.ny;
         uint4 r = border ? step_border_record() : step_record(0, 0);
         if (!border) r.w |= group_lod(0, 0) << 8;
@@ -221,7 +220,7 @@ __global__ __launch_bounds__(256) void sync_records_kernel(uint4* __restrict__ s
         const uint32_t s = rec_idx[i], n1 = (1u << st.shift_xz) - 1u;
         const uint4 r = rec[i];
         sec[s] = r;
-        const uint32_t X = (s & n1) + 4u, Z = ((s >> st.shift_xz) & n1) + 4u, Y = (s >> (2 * st.shift_xz)) + 4u;
+        const uint32_t X = (s & n1) + 1u, Z = ((s >> st.shift_xz) & n1) + 1u, Y = (s >> (2 * st.shift_xz)) + 1u;
         const uint64_t m = (uint64_t)r.x | (uint64_t)r.y << 32;
         st.steps[X + Z * st.step_z + Y * st.step_y] = step_record(m, r.z);
         st.masks[X + Z * st.step_z + Y * st.step_y] = mask_record(m, r.z, 0);
@@ -243,7 +242,7 @@ __global__ __launch_bounds__(256) void sync_groups_kernel(StepTables st, uint64_
         st.groups[gx + 1u + (gz + 1u) * st.group_z + (gy + 1u) * st.group_y] = m | st.outside;
     }
     if (((m | st.outside) >> b) & 1u) return;
-    const uint32_t X = gx * 4u + (b & 3u) + 4u, Z = gz * 4u + ((b >> 2) & 3u) + 4u, Y = gy * 4u + (b >> 4) + 4u;
+    const uint32_t X = gx * 4u + (b & 3u) + 1u, Z = gz * 4u + ((b >> 2) & 3u) + 1u, Y = gy * 4u + (b >> 4) + 1u;
     uint4 r = step_record(0, 0);
     r.w |= group_lod(m, b) << 8;
     st.steps[X + Z * st.step_z + Y * st.step_y] = r;
@@ -697,7 +696,7 @@ int vrt_world_create(const vrt_world_desc* desc, void* stream, vrt_world** out) 
             w->d_palette = (uint64_t*)(w->d_tables + o_palette);
             w->d_lut = (uint64_t*)(w->d_tables + o_lut);
             const WorldTables t{w->d_sec,       w->d_steps,     w->d_masks, w->d_groups, w->d_sgroups, w->d_palette,
-                                w->nsec,        w->step_z(),    w->step_y(), w->step_first(), w->step_n(),
+                                w->nsec,        w->step_z(),    w->step_y(), w->step_n(),
                                 1u << w->shift_xz, 1u << w->shift_y, (uint32_t)w->h_groups.size(),
                                 w->group_z(),   w->group_y(),   w->group_n(), w->group_outside()};
             const uint32_t n = std::max({w->nsec, w->step_n(), w->group_n(), 256u});
