@@ -33,6 +33,18 @@ __global__ __launch_bounds__(64) void load16_kernel(const void* table, uint32_t 
     out[k] = v;
 }
 
+// Thread m: the numbers of mantissa m, of both signs and exponents lo to hi, whose reciprocal differs.
+__global__ __launch_bounds__(256) void reciprocal_kernel(int lo, int hi, uint32_t* __restrict__ differ) {
+    const uint32_t m = blockIdx.x * 256 + threadIdx.x;
+    uint32_t bad = 0;
+    for (int e = lo; e <= hi; e++)
+        for (uint32_t s = 0; s < 2; s++) {
+            const float x = __uint_as_float(s << 31 | (uint32_t)(e + 127) << 23 | m);
+            bad += __float_as_uint(vrt::reciprocal_in_range(x)) != __float_as_uint(1.0f / x);
+        }
+    if (bad) atomicAdd(differ, bad);
+}
+
 }  // namespace
 
 extern "C" {
@@ -60,6 +72,12 @@ uint32_t check_launches(uint64_t blocks, uint32_t threads, uint32_t* each, uint3
     for (uint64_t first = 0; first < blocks && n < max; first += each[n++])
         each[n] = vrt::launch_blocks(blocks - first, threads);
     return n;
+}
+
+// -126 <= lo <= hi <= 127; differ: one count on the device, added to.
+int check_reciprocals(int lo, int hi, uint32_t* differ, void* stream) {
+    reciprocal_kernel<<<1u << 15, 256, 0, (hipStream_t)stream>>>(lo, hi, differ);
+    return (int)hipGetLastError();
 }
 
 }  // extern "C"

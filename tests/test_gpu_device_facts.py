@@ -18,6 +18,7 @@ def checks(cuda):
     P, u32 = C.c_void_p, C.c_uint32
     lib.check_structured_loads.argtypes = [P, u32, u32, P, u32, P, P]
     lib.check_take_slots.argtypes = [P, u32]
+    lib.check_reciprocals.argtypes = [C.c_int, C.c_int, P, P]
     return lib
 
 
@@ -48,6 +49,13 @@ def test_structured_loads_up_to_4_gib(checks):
     assert out.tolist() == [[1000003 * i + 19, -7 * i] for i in even] + [[0, 0]]
     del buf
     torch.cuda.empty_cache()
+
+
+def test_reciprocal_in_range(checks):
+    """reciprocal_in_range is 1 / x, correctly rounded, for every x with 2^-100 <= |x| < 2^101."""
+    differ = torch.zeros(1, dtype=torch.int32, device="cuda")
+    assert checks.check_reciprocals(-100, 100, differ.data_ptr(), torch.cuda.current_stream().cuda_stream) == 0
+    assert int(differ) == 0
 
 
 def test_worlds_past_the_reach_of_structured_loads(vrt, checks):
