@@ -80,7 +80,8 @@ typedef struct vrt_world_desc {
     uint32_t initial_slots;  /* device brick slots reserved up front (0 = grow on demand) */
     uint32_t max_slots;      /* slot arena capacity (0 = 128 per sector: twice the bricks the grid holds, so a
                                 sector's run of up to 64 slots can move even in a nearly full world; device
-                                memory follows the highest slot in use, not this bound); at most 2^28 */
+                                memory follows the highest slot in use, not this bound); at most 2^28.
+                                A world with memory for 2^26 slots or more (38.7 GB) is cast in a slower form */
 } vrt_world_desc;
 
 /* Shape of a created world (all derived from the descriptor). */

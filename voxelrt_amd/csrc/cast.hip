@@ -820,8 +820,8 @@ int vrt_cast_one_f64(const vrt_world* world, const double origin[3], const doubl
         if (!world || !origin || !dir || !out) return fail(VRT_ERR_INVALID_ARGUMENT, "vrt_cast_one_f64: null argument");
         if (int rcw = check_world(world, "vrt_cast_one_f64"); rcw != VRT_OK) return rcw;
         if (world->log2_y > 13) return fail(VRT_ERR_INVALID_ARGUMENT, "vrt_cast_one_f64: world taller than 8192 voxels");
-        // the loop has no exit for leaving the world (VoxelMap.cpp:140-170): every step up to the
-        // cap runs on one lane, so the cap is bounded like every other cast's
+        // the loop has no exit for leaving the world (VoxelMap.cpp:140-170): one wave makes every step
+        // up to the cap, so the cap is bounded like every other cast's
         if (max_iters == 0 || max_iters > 65535)
             return fail(VRT_ERR_INVALID_ARGUMENT, "vrt_cast_one_f64: max_iters must be 1..65535");
         // one pick of a world at a time: they share its result slot, and the null stream
